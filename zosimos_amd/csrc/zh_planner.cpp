@@ -1052,6 +1052,100 @@ static int warp_variant(const StageDesc& d, uint32_t flags) {
   return sep ? v + 1 : v;
 }
 
+// ---- any-format kernels (zh_any.hip) --------------------------------------------
+// Fields of the four components of a texel's code (demux, stage.frag:533-641):
+// {offset, width} or {constant} for width 0.
+static TableField component(uint32_t bits, uint32_t k) {
+  static const uint8_t F[18][4][2] = {
+      {{0, 8}, {0, 8}, {0, 8}, {0, 8}},       {{0, 2}, {2, 3}, {5, 3}, {1, 0}},
+      {{0, 3}, {3, 3}, {6, 2}, {1, 0}},       {},
+      {{0, 4}, {4, 4}, {8, 4}, {12, 4}},      {{0, 4}, {4, 4}, {8, 4}, {1, 0}},
+      {{4, 4}, {9, 4}, {12, 4}, {1, 0}},      {{0, 5}, {5, 6}, {11, 5}, {1, 0}},
+      {{0, 8}, {0, 0}, {0, 0}, {8, 8}},       {{0, 8}, {8, 8}, {16, 8}, {1, 0}},
+      {{0, 8}, {8, 8}, {16, 8}, {24, 8}},     {},
+      {},                                     {},
+      {{0, 2}, {2, 10}, {12, 10}, {22, 10}},  {{0, 10}, {10, 10}, {20, 10}, {30, 2}},
+      {{2, 10}, {12, 10}, {22, 10}, {1, 0}},  {{0, 10}, {10, 10}, {20, 10}, {1, 0}}};
+  const uint8_t* f = F[bits][k];
+  return f[1] ? TableField{f[0], f[1], 0, 0} : TableField{0, 0, f[0], 0};
+}
+
+// parts_normalize (stage.frag:654-747): per channel the component it takes
+// (0-3) or a constant (4: 0, 5: 1).
+static const uint8_t* normal_parts(uint32_t parts) {
+  static const uint8_t N[22][4] = {{4, 4, 4, 0}, {0, 4, 4, 5}, {4, 0, 4, 5}, {4, 4, 0, 5}, {0, 0, 0, 5}, {0, 0, 0, 3},
+                                   {0, 1, 2, 5}, {2, 1, 0, 5}, {0, 1, 2, 3}, {0, 1, 2, 5}, {0, 1, 2, 3}, {2, 1, 0, 5},
+                                   {1, 2, 3, 0}, {1, 2, 3, 5}, {3, 2, 1, 0}, {3, 2, 1, 5}, {5, 4, 4, 5}, {0, 1, 2, 5},
+                                   {0, 1, 2, 3}, {0, 1, 2, 5}, {0, 1, 2, 3}, {5, 4, 4, 5}};
+  return N[std::min(parts, 21u)];
+}
+
+static bool wide_bits(uint32_t bits) { return bits == 3 || (bits >= 11 && bits <= 13) || bits >= 18; }
+
+// The decode table of a load: colour channels of one width share a segment
+// (one transfer decodes all three), alpha has its own.
+static TableDesc decode_table(const Slot& s) {
+  TableDesc t{};
+  static const uint8_t kBgra[4] = {2, 1, 0, 3};  // native BGRA8 is swizzled, staged Bgra is not
+  const uint8_t* sel = s.native && s.parts == ZH_PARTS_BGRA ? kBgra : normal_parts(s.parts);
+  uint32_t at = 0;
+  for (uint32_t k = 0; k < 4; ++k) {
+    TableField f = sel[k] < 4 ? component(s.bits, sel[k]) : TableField{0, 0, (uint16_t)(sel[k] - 4), 0};
+    bool shared = false;
+    for (uint32_t j = 0; j < k && k < 3 && !shared; ++j)
+      if (t.ch[j].wd == f.wd && t.ch[j].cst == f.cst) {
+        f.off = t.ch[j].off;
+        shared = true;
+      }
+    if (!shared) {
+      f.off = (uint16_t)at;
+      at += 1u << f.wd;
+    }
+    t.ch[k] = f;
+  }
+  t.entries = at;
+  return t;
+}
+
+// Shape of the any-format kernels the pointwise program has (AnyShape), its
+// decode tables set; -1 for any other program.
+static int any_shape(StageDesc& d, bool flat) {
+  static const uint8_t kOver[6] = {OP_LOAD, OP_PREMUL, OP_LOAD, OP_PREMUL, OP_OVER, OP_UNPREMUL};
+  const uint32_t n = d.n_instr;
+  if (n < 2 || d.code[0].op != OP_LOAD || d.code[0].b) return -1;
+  uint32_t i = 1, shape = 0;
+  if (d.code[1].op == OP_PREMUL) {
+    if (n < 7) return -1;
+    for (uint32_t k = 0; k < 6; ++k)
+      if (d.code[k].op != kOver[k]) return -1;
+    if (!d.code[2].b) return -1;
+    shape = ANY_OVER;
+    i = 6;
+  }
+  if (d.code[i].op == OP_MAT3) ++i;
+  if (i + 1 != n || d.code[i].op != OP_STORE) return -1;
+  const uint64_t w = flat ? (uint64_t)d.width * d.height : d.width, h = flat ? 1 : d.height;
+  if ((w + kPix - 1) / kPix * h >= (1ull << 32)) return -1;
+  // LabLch mixes channels.  16-bit and float texels evaluate their transfer
+  // per pixel, narrower ones through a table when loaded.
+  auto power = [](const Slot& s) { return s.transfer <= 3 || (s.transfer >= 6 && s.transfer <= 8); };
+  auto fits = [&](const Slot& s) { return s.width == w && s.height == h && s.transfer != ZH_TRANSFER_LABLCH; };
+  for (uint32_t k = 0; k < 2; ++k) {
+    if (k == 1 && !(shape & ANY_OVER)) break;
+    const Slot& s = d.slot[d.code[2 * k].a];
+    if (!fits(s)) return -1;
+    uint32_t c = s.fmt == FMT_F16 ? SRC_F16 : s.fmt == FMT_F32 ? SRC_F32 : wide_bits(s.bits) ? SRC_WIDE : SRC_TABLE;
+    if (c == SRC_TABLE) d.table[k] = decode_table(s);
+    if (c == SRC_WIDE && power(s)) shape |= ANY_POW;
+    shape |= c << (2 + 2 * k);
+  }
+  const Slot& o = d.slot[d.code[n - 1].a];
+  if (!fits(o)) return -1;
+  const uint32_t c = o.native ? DST_U8 : o.fmt == FMT_F16 ? DST_F16 : o.fmt == FMT_F32 ? DST_F32 : wide_bits(o.bits) ? DST_WIDE : DST_CODE;
+  if (c >= DST_CODE && power(o)) shape |= ANY_POW;
+  return (int)(shape | c << 6);
+}
+
 bool warp_staged_fits(const StageDesc& d, uint32_t tw, uint32_t th) {
   if (d.kind != STAGE_RESAMPLE || d.variant < 0 || !(d.variant & 1) || d.n_layers != 1) return false;
   const bool has = d.variant >= kJitWarpBase ? jit_warp_has_staged((d.variant - kJitWarpBase) / 2)
@@ -1449,6 +1543,7 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
           s.row_stride = (uint64_t)s.width * s.bpp;
         }
       }
+      sp.any = any_shape(sp.desc, flat);
       for (size_t k = 0; k < sp.slot_ref.size(); ++k)
         if (sp.slot_ref[k] > -1000000 || sp.slot_ref[k] < -2000000000ll) {
           // quantisation-only slots (strict mode) carry no traffic
@@ -1466,6 +1561,8 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
         t << " [kernel jit#" << sp.jit << "]";
       else if (sp.fast)
         t << " [kernel interp-inline]";
+      else if (sp.any >= 0)
+        t << " [any-format kernel]";
       sp.text = t.str();
       plan.stages.push_back(sp);
       continue;

@@ -23,6 +23,8 @@
 extern "C" {
 hipError_t zh_launch_pointwise(const zh::StageDesc* d_dev, uint32_t width, uint32_t height, int flat, int fast,
                                uint32_t cus, hipStream_t stream);
+hipError_t zh_launch_any(uint32_t shape, const zh::StageDesc* d_dev, uint32_t width, uint32_t height, int flat,
+                         uint32_t cus, hipStream_t stream);
 hipError_t zh_launch_spec(int index, const zh::StageDesc* d_dev, uint32_t width, uint32_t height,
                           uint32_t cus, hipStream_t stream);
 hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, uint32_t cus,
@@ -1067,7 +1069,11 @@ static zh_status bind(zh_program* p, const zh_binding* b, uint32_t n) {
         for (size_t k = 0; k < refs.size(); ++k) aligned = aligned && d.slot[k].vec_ok;
         const StagePlan& sp = plan.stages[s];
         const bool jit = sp.jit >= 0 && s < p->jit_stage_fn.size() && p->jit_stage_fn[s];
-        variant[s] = !aligned ? 0 : sp.spec >= 0 ? 2 : jit ? 6 : sp.fast ? 1 : 0;
+        // The any-format kernels move groups as dwords.
+        bool words = sp.any >= 0;
+        for (size_t k = 0; k < refs.size(); ++k)
+          words = words && d.slot[k].ptr % 4 == 0 && (d.flat || d.slot[k].row_stride % 4 == 0);
+        variant[s] = aligned && sp.spec >= 0 ? 2 : aligned && jit ? 6 : words ? 7 : aligned && sp.fast ? 1 : 0;
       }
     }
     p->h_stages[s] = d;
@@ -1176,6 +1182,8 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
                                   (uint32_t)p->ctx->cus, s));
       else if (v == 2)
         ZH_HIP(zh_launch_spec(sp.spec, d, sp.desc.width, sp.desc.height, (uint32_t)p->ctx->cus, s));
+      else if (v == 7)
+        ZH_HIP(zh_launch_any((uint32_t)sp.any, d, sp.desc.width, sp.desc.height, (int)sp.desc.flat, (uint32_t)p->ctx->cus, s));
       else if (v == 6) {
         // A run-time kernel: the persistent grid of zh_launch_spec.
         const uint64_t groups = ((uint64_t)sp.desc.width * sp.desc.height + kPix - 1) / kPix;

@@ -140,6 +140,45 @@ struct Layer {
 
 enum StageKind : uint32_t { STAGE_POINTWISE = 0, STAGE_RESAMPLE = 1, STAGE_COPY = 2, STAGE_DYNAMIC = 3 };
 
+// Shape of a pointwise stage the any-format kernels run (zh_any.hip): a
+// program [load (mat3) store] or [load premul load premul over unpremul (mat3)
+// store] and the classes of its slots.
+//   bit 0: the 'over' of two loads; bit 1: a transfer of power functions
+//   evaluated per pixel; bits 2-3, 4-5: SrcClass of the loads; bits 6-8:
+//   DstClass.
+enum AnyShape : uint32_t { ANY_OVER = 1, ANY_POW = 2 };
+constexpr uint32_t kAnyShapes = 512;
+constexpr uint32_t any_src(uint32_t shape, uint32_t k) { return (shape >> (2 + 2 * k)) & 3u; }
+constexpr uint32_t any_dst(uint32_t shape) { return (shape >> 6) & 7u; }
+// Classes of loads and stores the any-format kernels are instantiated for.
+enum SrcClass : int {
+  SRC_TABLE = 0,  // integer texels of up to 10 bits per channel: decoded through a table
+  SRC_F16 = 1,    // linear RGBA16F
+  SRC_F32 = 2,    // linear RGBA32F
+  SRC_WIDE = 3,   // 16-bit channels; float texels with other parts or transfers
+  SRC_ANY = 4,    // (kernels only) any of them, by the slot
+};
+enum DstClass : int {
+  DST_U8 = 0,    // native RGBA8 / BGRA8
+  DST_F16 = 1,   // linear RGBA16F
+  DST_F32 = 2,   // linear RGBA32F
+  DST_CODE = 3,  // integer texels of up to 10 bits per channel
+  DST_WIDE = 4,  // every other format, as SRC_WIDE
+};
+
+// How the decode table of an any-format kernel's load is laid out (SRC_TABLE
+// of zh_any.h): the bit field of each channel in the texel's code, and the
+// channel's segment of the table.
+struct TableField {
+  uint16_t sh, wd;   // bit offset and width; width 0: the constant `cst`
+  uint16_t cst, off; // off: first entry of the segment
+};
+struct TableDesc {
+  TableField ch[4];  // r, g, b, a
+  uint32_t entries;
+  uint32_t pad;
+};
+
 struct StageDesc {
   uint32_t kind;
   uint32_t width, height;     // output grid
@@ -163,6 +202,7 @@ struct StageDesc {
   // meets the tile, four tiles per word (bit l: layer l); null: the kernel
   // tests each layer itself.
   const uint32_t* tile_layers;
+  TableDesc table[2];         // any-format kernels: the decode tables of their loads
   uint32_t* error_flag;       // set to 1 by a kernel that met an impossible case
   Layer layer[kMaxLayers];
   Slot slot[kMaxSlots];
