@@ -20,6 +20,7 @@ LIB = os.path.join(HERE, "libzosimos_hip.so")
 SOURCES = [
     "zh_kernels.hip",
     "zh_any.hip",
+    "zh_field.hip",
     "zh_spec.hip",
     "zh_warp.hip",
     "zh_mlp.hip",
@@ -31,7 +32,7 @@ SOURCES = [
     "zh_dynamic.cpp",
     "zh_jit.cpp",
 ]
-HEADERS = ["zh_stage.h", "zh_codec.h", "zh_device.h", "zh_any.h", "zh_spec.h", "zh_prog.h", "zh_spec_kernels.h",
+HEADERS = ["zh_stage.h", "zh_codec.h", "zh_device.h", "zh_any.h", "zh_field.h", "zh_spec.h", "zh_prog.h", "zh_spec_kernels.h",
            "zh_warp_kernels.h", "zh_internal.h",
            "zh_mlp.h"]
 ARCH = "gfx950"

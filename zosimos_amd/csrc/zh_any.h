@@ -21,9 +21,8 @@
 namespace zh {
 namespace any {
 
-// Groups move as dwords at any 4-byte aligned address (the row pitch and the
-// image address need no more; a group of kPix texels is a whole number of
-// dwords in every format).
+// Groups move as dwords wherever their address is a multiple of 4 (a group of
+// kPix texels is a whole number of dwords in every format).
 typedef uint32_t w2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t w3 __attribute__((ext_vector_type(3), aligned(4)));
 typedef uint32_t w4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -47,12 +46,39 @@ __device__ __forceinline__ float4 f4_bits(w4 v) {
   return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
 }
 
-// The group's texels at q: all kPix, or (a row's last group) the first n >= 1
-// one by one.  16-byte texels have no codes: load_floats reads them.
+// One texel's code (bpp 1, 3 at any address, 2 and 6 at even ones, 4 and 8 at
+// multiples of 4).
+__device__ __forceinline__ void load_code(const gbyte* p, uint32_t bpp, uint32_t& lo, uint32_t& hi) {
+  hi = 0u;
+  switch (bpp) {  // uniform
+    case 1: lo = gld<uint8_t>(p); break;
+    case 2: lo = gld<uint16_t>(p); break;
+    case 3:
+      lo = (uint32_t)gld<uint8_t>(p) | ((uint32_t)gld<uint8_t>(p + 1) << 8) | ((uint32_t)gld<uint8_t>(p + 2) << 16);
+      break;
+    case 4: lo = gld<uint32_t>(p); break;
+    case 6:
+      lo = (uint32_t)gld<uint16_t>(p) | ((uint32_t)gld<uint16_t>(p + 2) << 16);
+      hi = gld<uint16_t>(p + 4);
+      break;
+    case 8: {
+      const w2 v = gld<w2>(p);
+      lo = v.x;
+      hi = v.y;
+      break;
+    }
+    default: lo = 0u;
+  }
+}
+
+// The group's texels at q: all kPix by dwords, or one by one where the group is
+// a row's last (its first n >= 1 texels; the others repeat the last one and
+// their results are not stored) or its address is no multiple of 4.  16-byte
+// texels have no codes: load_floats reads them.
 __device__ __forceinline__ void load_group(const gbyte* q, uint32_t bpp, int n, Codes& c) {
 #pragma unroll
   for (int i = 0; i < kPix; ++i) c.lo[i] = c.hi[i] = 0u;
-  if (n == kPix) {
+  if (n == kPix && ((uintptr_t)q & 3u) == 0) {
     switch (bpp) {  // uniform
       case 1: {
         const uint32_t v = nt_get<uint32_t>(q);
@@ -112,29 +138,8 @@ __device__ __forceinline__ void load_group(const gbyte* q, uint32_t bpp, int n, 
       default: break;
     }
   } else {
-    // Texels past the end repeat the last one (their results are not stored).
 #pragma unroll
-    for (int i = 0; i < kPix; ++i) {
-      const gbyte* p = q + (uint32_t)min(i, n - 1) * bpp;
-      switch (bpp) {  // uniform
-        case 1: c.lo[i] = gld<uint8_t>(p); break;
-        case 2: c.lo[i] = gld<uint16_t>(p); break;
-        case 3: c.lo[i] = (uint32_t)gld<uint8_t>(p) | ((uint32_t)gld<uint8_t>(p + 1) << 8) |
-                          ((uint32_t)gld<uint8_t>(p + 2) << 16); break;
-        case 4: c.lo[i] = gld<uint32_t>(p); break;
-        case 6:
-          c.lo[i] = (uint32_t)gld<uint16_t>(p) | ((uint32_t)gld<uint16_t>(p + 2) << 16);
-          c.hi[i] = gld<uint16_t>(p + 4);
-          break;
-        case 8: {
-          const w2 v = gld<w2>(p);
-          c.lo[i] = v.x;
-          c.hi[i] = v.y;
-          break;
-        }
-        default: break;
-      }
-    }
+    for (int i = 0; i < kPix; ++i) load_code(q + (uint32_t)min(i, n - 1) * bpp, bpp, c.lo[i], c.hi[i]);
   }
 }
 
@@ -168,7 +173,7 @@ __device__ __forceinline__ void store_group(gbyte* q, uint32_t bpp, int n, const
   // into one from a variable index and c ends up in memory.
   const uint32_t l0 = c.lo[0], l1 = c.lo[1], l2 = c.lo[2], l3 = c.lo[3];
   const uint32_t h0 = c.hi[0], h1 = c.hi[1], h2 = c.hi[2], h3 = c.hi[3];
-  if (n == kPix) {
+  if (n == kPix && ((uintptr_t)q & 3u) == 0) {
     switch (bpp) {  // uniform
       case 1: nt_put<uint32_t>(q, l0 | (l1 << 8) | (l2 << 16) | (l3 << 24)); break;
       case 2: nt_put<w2>(q, w2{l0 | (l1 << 16), l2 | (l3 << 16)}); break;
@@ -187,13 +192,13 @@ __device__ __forceinline__ void store_group(gbyte* q, uint32_t bpp, int n, const
       default: break;
     }
   } else {
-    // 1 <= n < kPix
-    store_code(q, bpp, l0, h0);
+    store_code(q, bpp, l0, h0);  // n >= 1
     if (n > 1) store_code(q + bpp, bpp, l1, h1);
     if (n > 2) store_code(q + 2 * bpp, bpp, l2, h2);
+    if (n > 3) store_code(q + 3 * bpp, bpp, l3, h3);
   }
 }
-static_assert(kPix == 4, "partial groups hold up to 3 texels");
+static_assert(kPix == 4, "a group holds 4 texels");
 
 __device__ __forceinline__ void store_floats(gbyte* q, int n, const Px& X) {
   w4 v[kPix];
@@ -318,26 +323,21 @@ __device__ __forceinline__ void fill_table(const Src& s, CDesc d, float* tab) {
   if constexpr (S != SRC_TABLE && S != SRC_ANY) return;
   if (S == SRC_ANY && is_wide(s.bits)) return;  // uniform
   const float* dec = reinterpret_cast<const Luts*>(d->srgb_lut)->dec;
-  for (uint32_t e = threadIdx.x; e < s.t.entries; e += kBlock) {
-    // The channel whose segment holds entry e: the last one to start at or
-    // before it (colour channels may share a segment; alpha has its own).
-    uint32_t k = 0;
-    TableField f = s.t.ch[0];
 #pragma unroll
-    for (uint32_t c = 1; c < 4; ++c)
-      if (s.t.ch[c].off <= e && s.t.ch[c].off >= f.off) {
-        k = c;
-        f = s.t.ch[c];
+  for (int k = 0; k < 4; ++k) {
+    const TableChannel c = s.t.ch[k];
+    if (!(c.flags & TABLE_OWNER)) continue;  // uniform
+    const uint32_t n = c.mask / 4 + 1;
+    for (uint32_t code = threadIdx.x; code < n; code += kBlock) {
+      float v;
+      if (s.native) {
+        v = k < 3 && s.transfer == 5 ? dec[code] : (float)code * (1.0f / 255.0f);
+      } else {
+        v = n > 1 ? fd(code, (float)(n - 1)) : (c.flags & TABLE_ONE) ? 1.0f : 0.0f;
+        if (k < 3) v = untransfer1(v, s.transfer);
       }
-    const uint32_t code = e - f.off;
-    float v;
-    if (s.native) {
-      v = k < 3 && s.transfer == 5 ? dec[code] : (float)code * (1.0f / 255.0f);
-    } else {
-      v = f.wd ? fd(code, (float)((1u << f.wd) - 1u)) : (float)f.cst;
-      if (k < 3) v = untransfer1(v, s.transfer);
+      tab[c.base / 4 + code] = v;
     }
-    tab[e] = v;
   }
 }
 
@@ -360,7 +360,10 @@ __device__ __forceinline__ void table_group(const TableDesc& t, const Codes& c, 
   for (int i = 0; i < kPix; ++i) {
     float v[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = tab[t.ch[k].off + ((c.lo[i] >> t.ch[k].sh) & ((1u << t.ch[k].wd) - 1u))];
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t at = (__builtin_amdgcn_alignbit(c.lo[i], c.lo[i], t.ch[k].rot) & t.ch[k].mask) | t.ch[k].base;
+      v[k] = *(const float*)((const char*)tab + at);
+    }
     X[i] = make_float4(v[0], v[1], v[2], v[3]);
   }
 }
@@ -387,24 +390,31 @@ __device__ __forceinline__ void wide_group(const Src& s, const Codes& c, Px& X) 
   untransfer_group<POW>(X, s.transfer);
 }
 
-// X of the fetched group (16-byte texels are read here, at q).
+// X of a group's codes (16-byte texels: of the floats in X).
 template <int S, bool POW>
-__device__ __forceinline__ void decode_group(const Src& s, const gbyte* q, int n, const Codes& c, Px& X,
-                                             const float* tab) {
+__device__ __forceinline__ void decode_codes(const Src& s, const Codes& c, Px& X, const float* tab) {
   if constexpr (S == SRC_TABLE) {
     table_group(s.t, c, X, tab);
   } else if constexpr (S == SRC_F16) {
 #pragma unroll
     for (int i = 0; i < kPix; ++i) X[i] = dec_f16(c.lo[i], c.hi[i]);
-  } else if constexpr (S == SRC_F32) {
-    load_floats(q, n, X);
-  } else if (S == SRC_ANY && !is_wide(s.bits)) {  // uniform
-    table_group(s.t, c, X, tab);
-  } else {
-    if (s.bits == 19) load_floats(q, n, X);
-    wide_group<POW>(s, c, X);
+  } else if constexpr (S != SRC_F32) {
+    if (S == SRC_ANY && !is_wide(s.bits)) table_group(s.t, c, X, tab);  // uniform
+    else wide_group<POW>(s, c, X);
   }
 }
+
+// X of the fetched group at q (16-byte texels are read here).
+template <int S, bool POW>
+__device__ __forceinline__ void decode_group(const Src& s, const gbyte* q, int n, const Codes& c, Px& X,
+                                             const float* tab) {
+  if (S == SRC_F32 || (S >= SRC_WIDE && s.bits == 19)) load_floats(q, n, X);
+  decode_codes<S, POW>(s, c, X, tab);
+}
+
+template <bool WITH> struct LutOf { typedef uint32_t type; };
+template <> struct LutOf<true> { typedef Luts type; };
+constexpr bool has_table(int s) { return s == SRC_TABLE || s == SRC_ANY; }
 
 // ---- encode --------------------------------------------------------------------
 struct Dst {

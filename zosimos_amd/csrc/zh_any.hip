@@ -69,10 +69,6 @@ __device__ __forceinline__ void colour(const Src& a, const Src& b, bool mat, con
   }
 }
 
-template <bool WITH> struct LutOf { typedef uint32_t type; };
-template <> struct LutOf<true> { typedef Luts type; };
-constexpr bool has_table(int s) { return s == SRC_TABLE || s == SRC_ANY; }
-
 // A persistent grid striding over the stage's groups of kPix texels: the
 // whole image as one row when every slot is tight (flat), else
 // ceil(width / kPix) groups a row, the last of a row partial.  A lane's next

@@ -1053,10 +1053,13 @@ static int warp_variant(const StageDesc& d, uint32_t flags) {
 }
 
 // ---- any-format kernels (zh_any.hip) --------------------------------------------
-// Fields of the four components of a texel's code (demux, stage.frag:533-641):
-// {offset, width} or {constant} for width 0.
-static TableField component(uint32_t bits, uint32_t k) {
-  static const uint8_t F[18][4][2] = {
+// A component of a texel's code (demux, stage.frag:533-641): bit offset and
+// width, or (width 0) the constant `sh`.
+struct Field {
+  uint8_t sh, wd;
+};
+static Field component(uint32_t bits, uint32_t k) {
+  static const Field F[18][4] = {
       {{0, 8}, {0, 8}, {0, 8}, {0, 8}},       {{0, 2}, {2, 3}, {5, 3}, {1, 0}},
       {{0, 3}, {3, 3}, {6, 2}, {1, 0}},       {},
       {{0, 4}, {4, 4}, {8, 4}, {12, 4}},      {{0, 4}, {4, 4}, {8, 4}, {1, 0}},
@@ -1066,8 +1069,7 @@ static TableField component(uint32_t bits, uint32_t k) {
       {},                                     {},
       {{0, 2}, {2, 10}, {12, 10}, {22, 10}},  {{0, 10}, {10, 10}, {20, 10}, {30, 2}},
       {{2, 10}, {12, 10}, {22, 10}, {1, 0}},  {{0, 10}, {10, 10}, {20, 10}, {1, 0}}};
-  const uint8_t* f = F[bits][k];
-  return f[1] ? TableField{f[0], f[1], 0, 0} : TableField{0, 0, f[0], 0};
+  return F[bits][k];
 }
 
 // parts_normalize (stage.frag:654-747): per channel the component it takes
@@ -1083,28 +1085,83 @@ static const uint8_t* normal_parts(uint32_t parts) {
 static bool wide_bits(uint32_t bits) { return bits == 3 || (bits >= 11 && bits <= 13) || bits >= 18; }
 
 // The decode table of a load: colour channels of one width share a segment
-// (one transfer decodes all three), alpha has its own.
+// (one transfer decodes all three), alpha has its own; the widest segments
+// come first, so each lies at a multiple of its size.
 static TableDesc decode_table(const Slot& s) {
   TableDesc t{};
   static const uint8_t kBgra[4] = {2, 1, 0, 3};  // native BGRA8 is swizzled, staged Bgra is not
   const uint8_t* sel = s.native && s.parts == ZH_PARTS_BGRA ? kBgra : normal_parts(s.parts);
+  Field f[4];
+  for (uint32_t k = 0; k < 4; ++k) f[k] = sel[k] < 4 ? component(s.bits, sel[k]) : Field{(uint8_t)(sel[k] - 4), 0};
   uint32_t at = 0;
-  for (uint32_t k = 0; k < 4; ++k) {
-    TableField f = sel[k] < 4 ? component(s.bits, sel[k]) : TableField{0, 0, (uint16_t)(sel[k] - 4), 0};
-    bool shared = false;
-    for (uint32_t j = 0; j < k && k < 3 && !shared; ++j)
-      if (t.ch[j].wd == f.wd && t.ch[j].cst == f.cst) {
-        f.off = t.ch[j].off;
-        shared = true;
-      }
-    if (!shared) {
-      f.off = (uint16_t)at;
-      at += 1u << f.wd;
+  for (int wd = 10; wd >= 0; --wd)
+    for (uint32_t k = 0; k < 4; ++k) {
+      if (f[k].wd != wd) continue;
+      TableChannel& c = t.ch[k];
+      c.mask = ((1u << wd) - 1u) * 4;
+      c.rot = wd ? (f[k].sh + 30u) % 32u : 0u;
+      bool shared = false;
+      for (uint32_t j = 0; j < k && k < 3 && !shared; ++j)
+        if (f[j].wd == wd && (wd || f[j].sh == f[k].sh)) {
+          c.base = t.ch[j].base;
+          shared = true;
+        }
+      if (shared) continue;
+      c.base = at;
+      c.flags = TABLE_OWNER | (!wd && f[k].sh ? TABLE_ONE : 0u);
+      at += (1u << wd) * 4;
     }
-    t.ch[k] = f;
-  }
-  t.entries = at;
   return t;
+}
+
+static bool power_transfer(const Slot& s) { return s.transfer <= 3 || (s.transfer >= 6 && s.transfer <= 8); }
+static uint32_t src_class(const Slot& s) {
+  return s.fmt == FMT_F16 ? SRC_F16 : s.fmt == FMT_F32 ? SRC_F32 : wide_bits(s.bits) ? SRC_WIDE : SRC_TABLE;
+}
+static uint32_t dst_class(const Slot& s) {
+  return s.native ? DST_U8 : s.fmt == FMT_F16 ? DST_F16 : s.fmt == FMT_F32 ? DST_F32 : wide_bits(s.bits) ? DST_WIDE
+                                                                                                       : DST_CODE;
+}
+
+// Shape of the kernels of zh_field.hip a 2-D pointwise program has, its decode
+// table set; -1 for any other program.
+static int field_shape(StageDesc& d) {
+  const uint32_t n = d.n_instr;
+  if (n < 2 || d.code[0].b || d.code[n - 1].op != OP_STORE) return -1;
+  if ((uint64_t)((d.width + kPix - 1) / kPix) * d.height >= (1ull << 32) - kBlock) return -1;
+  const Slot& o = d.slot[d.code[n - 1].a];
+  if (o.width != d.width || o.height != d.height || o.transfer == ZH_TRANSFER_LABLCH) return -1;
+  const uint32_t dst = dst_class(o);
+  uint32_t shape = dst << 6 | (dst >= DST_CODE && power_transfer(o) ? ANY_POW : 0u);
+  int read = -1;  // the slot sampled
+  if (n == 2 && d.code[0].op == OP_BOX3) {
+    shape |= FIELD_BOX3 << 9;
+    read = d.code[0].a;
+    if (d.slot[read].width != d.width || d.slot[read].height != d.height) return -1;
+  } else if (n == 2 && d.code[0].op == OP_NOISE) {
+    shape |= FIELD_NOISE << 9;
+  } else if (n == 2 && d.code[0].op == OP_GRID) {
+    shape |= FIELD_GRID << 9;
+  } else if (n == 2 && d.code[0].op == OP_NORMAL2D) {
+    shape |= FIELD_NORMAL << 9;
+  } else if (n == 4 && d.code[0].op == OP_GRID && d.code[1].op == OP_QUANT && d.code[2].op == OP_PALETTE) {
+    const Slot& qs = d.slot[d.code[1].a];
+    if (qs.bits != ZH_BITS_INT8X4 || qs.native || qs.transfer != ZH_TRANSFER_LINEAR ||
+        (qs.parts != ZH_PARTS_RGBA && qs.parts != 18 && qs.parts != ZH_PARTS_LCHA))
+      return -1;
+    shape |= FIELD_LOOKUP << 9;
+    read = d.code[2].a;
+  } else {
+    return -1;
+  }
+  if (read >= 0) {
+    const Slot& s = d.slot[read];
+    if (s.transfer == ZH_TRANSFER_LABLCH) return -1;
+    const uint32_t c = src_class(s);
+    if (c == SRC_TABLE) d.table[0] = decode_table(s);
+    shape |= c << 2;
+  }
+  return (int)shape;
 }
 
 // Shape of the any-format kernels the pointwise program has (AnyShape), its
@@ -1128,21 +1185,20 @@ static int any_shape(StageDesc& d, bool flat) {
   if ((w + kPix - 1) / kPix * h >= (1ull << 32)) return -1;
   // LabLch mixes channels.  16-bit and float texels evaluate their transfer
   // per pixel, narrower ones through a table when loaded.
-  auto power = [](const Slot& s) { return s.transfer <= 3 || (s.transfer >= 6 && s.transfer <= 8); };
   auto fits = [&](const Slot& s) { return s.width == w && s.height == h && s.transfer != ZH_TRANSFER_LABLCH; };
   for (uint32_t k = 0; k < 2; ++k) {
     if (k == 1 && !(shape & ANY_OVER)) break;
     const Slot& s = d.slot[d.code[2 * k].a];
     if (!fits(s)) return -1;
-    uint32_t c = s.fmt == FMT_F16 ? SRC_F16 : s.fmt == FMT_F32 ? SRC_F32 : wide_bits(s.bits) ? SRC_WIDE : SRC_TABLE;
+    const uint32_t c = src_class(s);
     if (c == SRC_TABLE) d.table[k] = decode_table(s);
-    if (c == SRC_WIDE && power(s)) shape |= ANY_POW;
+    if (c == SRC_WIDE && power_transfer(s)) shape |= ANY_POW;
     shape |= c << (2 + 2 * k);
   }
   const Slot& o = d.slot[d.code[n - 1].a];
   if (!fits(o)) return -1;
-  const uint32_t c = o.native ? DST_U8 : o.fmt == FMT_F16 ? DST_F16 : o.fmt == FMT_F32 ? DST_F32 : wide_bits(o.bits) ? DST_WIDE : DST_CODE;
-  if (c >= DST_CODE && power(o)) shape |= ANY_POW;
+  const uint32_t c = dst_class(o);
+  if (c >= DST_CODE && power_transfer(o)) shape |= ANY_POW;
   return (int)(shape | c << 6);
 }
 
@@ -1544,6 +1600,7 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
         }
       }
       sp.any = any_shape(sp.desc, flat);
+      if (!flat && sp.any < 0) sp.field = field_shape(sp.desc);
       for (size_t k = 0; k < sp.slot_ref.size(); ++k)
         if (sp.slot_ref[k] > -1000000 || sp.slot_ref[k] < -2000000000ll) {
           // quantisation-only slots (strict mode) carry no traffic
@@ -1563,6 +1620,8 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
         t << " [kernel interp-inline]";
       else if (sp.any >= 0)
         t << " [any-format kernel]";
+      else if (sp.field >= 0)
+        t << " [field kernel]";
       sp.text = t.str();
       plan.stages.push_back(sp);
       continue;

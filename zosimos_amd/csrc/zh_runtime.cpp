@@ -25,6 +25,8 @@ hipError_t zh_launch_pointwise(const zh::StageDesc* d_dev, uint32_t width, uint3
                                uint32_t cus, hipStream_t stream);
 hipError_t zh_launch_any(uint32_t shape, const zh::StageDesc* d_dev, uint32_t width, uint32_t height, int flat,
                          uint32_t cus, hipStream_t stream);
+hipError_t zh_launch_field(uint32_t shape, const zh::StageDesc* d_dev, uint32_t width, uint32_t height, uint32_t cus,
+                           hipStream_t stream);
 hipError_t zh_launch_spec(int index, const zh::StageDesc* d_dev, uint32_t width, uint32_t height,
                           uint32_t cus, hipStream_t stream);
 hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, uint32_t cus,
@@ -929,7 +931,7 @@ zh_status zh_program_set_knob(zh_program* p, int32_t knob, const void* data, uin
     const StagePlan& b = p->plan.stages[i];
     same = a.desc.kind == b.desc.kind && a.tile_mode == b.tile_mode && a.desc.tiles_x == b.desc.tiles_x &&
            a.desc.tiles_y == b.desc.tiles_y && a.slot_ref == b.slot_ref && a.lds_bytes <= b.lds_bytes &&
-           a.spec == b.spec && a.jit == b.jit && a.fast == b.fast && a.desc.flat == b.desc.flat &&
+           a.spec == b.spec && a.jit == b.jit && a.any == b.any && a.field == b.field && a.fast == b.fast && a.desc.flat == b.desc.flat &&
            a.desc.variant == b.desc.variant && a.staged == b.staged;
   }
   p->params = params;
@@ -1069,11 +1071,15 @@ static zh_status bind(zh_program* p, const zh_binding* b, uint32_t n) {
         for (size_t k = 0; k < refs.size(); ++k) aligned = aligned && d.slot[k].vec_ok;
         const StagePlan& sp = plan.stages[s];
         const bool jit = sp.jit >= 0 && s < p->jit_stage_fn.size() && p->jit_stage_fn[s];
-        // The any-format kernels move groups as dwords.
-        bool words = sp.any >= 0;
-        for (size_t k = 0; k < refs.size(); ++k)
-          words = words && d.slot[k].ptr % 4 == 0 && (d.flat || d.slot[k].row_stride % 4 == 0);
-        variant[s] = aligned && sp.spec >= 0 ? 2 : aligned && jit ? 6 : words ? 7 : aligned && sp.fast ? 1 : 0;
+        // The any-format and field kernels address texels at their natural
+        // alignment (4 bytes at most).
+        bool natural = true;
+        for (size_t k = 0; k < refs.size(); ++k) {
+          const uint32_t bpp = d.slot[k].bpp, align = bpp == 1 || bpp == 3 ? 1u : bpp == 2 || bpp == 6 ? 2u : 4u;
+          natural = natural && d.slot[k].ptr % align == 0 && (d.flat || d.slot[k].row_stride % align == 0);
+        }
+        variant[s] = aligned && sp.spec >= 0 ? 2 : aligned && jit ? 6 : natural && sp.any >= 0 ? 7
+                     : natural && sp.field >= 0 ? 8 : aligned && sp.fast ? 1 : 0;
       }
     }
     p->h_stages[s] = d;
@@ -1184,6 +1190,8 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
         ZH_HIP(zh_launch_spec(sp.spec, d, sp.desc.width, sp.desc.height, (uint32_t)p->ctx->cus, s));
       else if (v == 7)
         ZH_HIP(zh_launch_any((uint32_t)sp.any, d, sp.desc.width, sp.desc.height, (int)sp.desc.flat, (uint32_t)p->ctx->cus, s));
+      else if (v == 8)
+        ZH_HIP(zh_launch_field((uint32_t)sp.field, d, sp.desc.width, sp.desc.height, (uint32_t)p->ctx->cus, s));
       else if (v == 6) {
         // A run-time kernel: the persistent grid of zh_launch_spec.
         const uint64_t groups = ((uint64_t)sp.desc.width * sp.desc.height + kPix - 1) / kPix;

@@ -166,18 +166,34 @@ enum DstClass : int {
   DST_WIDE = 4,  // every other format, as SRC_WIDE
 };
 
+// Shape of a stage of zh_field.hip: bits 0-1 and 6-8 as AnyShape (no 'over'),
+// bits 2-3 the SrcClass of the image read, bits 9-11 the kind.
+enum FieldKind : uint32_t {
+  FIELD_BOX3 = 0,    // [box3 store]
+  FIELD_NOISE = 1,   // [noise store]
+  FIELD_GRID = 2,    // [grid store]
+  FIELD_NORMAL = 3,  // [normal2d store]
+  FIELD_LOOKUP = 4,  // [grid quant palette store], the quantisation through linear RGBA8
+};
+constexpr uint32_t kFieldShapes = 4096;
+constexpr uint32_t field_kind(uint32_t shape) { return shape >> 9; }
+
 // How the decode table of an any-format kernel's load is laid out (SRC_TABLE
-// of zh_any.h): the bit field of each channel in the texel's code, and the
-// channel's segment of the table.
-struct TableField {
-  uint16_t sh, wd;   // bit offset and width; width 0: the constant `cst`
-  uint16_t cst, off; // off: first entry of the segment
+// of zh_any.h).  A channel's entry is found by rotating the texel's code right
+// by `rot`, masking it and or-ing in the segment's byte offset: segments lie at
+// multiples of their size.
+struct TableChannel {
+  uint32_t rot;   // offset of the channel's bit field, less 2 (entries are 4 bytes), modulo 32
+  uint32_t mask;  // (entries - 1) * 4
+  uint32_t base;  // byte offset of the segment
+  // Bit 0: the channel fills its segment (others share it); bit 1: a field of
+  // no bits holds 1 instead of 0.
+  uint32_t flags;
 };
 struct TableDesc {
-  TableField ch[4];  // r, g, b, a
-  uint32_t entries;
-  uint32_t pad;
+  TableChannel ch[4];  // r, g, b, a
 };
+enum TableFlags : uint32_t { TABLE_OWNER = 1, TABLE_ONE = 2 };
 
 struct StageDesc {
   uint32_t kind;
