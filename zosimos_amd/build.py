@@ -21,6 +21,7 @@ SOURCES = [
     "zh_kernels.hip",
     "zh_any.hip",
     "zh_field.hip",
+    "zh_move.hip",
     "zh_spec.hip",
     "zh_warp.hip",
     "zh_mlp.hip",

@@ -111,6 +111,7 @@ struct StagePlan {
   int jit = -1;                   // pointwise: run-time kernel of the signature (zh_jit.cpp), -1 = none
   int any = -1;                   // pointwise: shape of the any-format kernels (zh_any.hip), -1 = none
   int field = -1;                 // pointwise: shape of the kernels of zh_field.hip, -1 = none
+  int move = 0;                   // resample: 32-bit words of a texel k_move moves (zh_move.hip), 0 = not its form
   bool staged = false;            // warp: the LDS-staged kernel (staged_tile), the box fitting its tile
   uint32_t lds_bytes = 0;
   uint64_t alg_bytes = 0;         // algorithmic HBM bytes (reads once + writes once)
@@ -236,7 +237,8 @@ struct zh_program {
   // Kernel per stage for the bound images: 0 general interpreter, 1
   // interpreter with in-line codecs, 2 specialised pointwise, 3 warp, 5 the
   // learned surrogate, 6 run-time pointwise, 7 any-format, 8 filter or
-  // generator (an image the faster kernel cannot address forces 7, 1 or 0).
+  // generator, 9 texel moves (an image the faster kernel cannot address forces
+  // 7, 1 or 0).
   std::vector<int> variant;
   // Learned colour surrogates per stage (zh_surrogate.cpp): packed matrix-core
   // operands (nullptr = none), the lattice check's verdict, master weights.

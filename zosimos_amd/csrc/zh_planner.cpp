@@ -1123,6 +1123,33 @@ static uint32_t dst_class(const Slot& s) {
                                                                                                        : DST_CODE;
 }
 
+// 32-bit words of a texel when the resample stage only moves texels
+// (zh_move.hip): nearest replacing paints through affine maps over a loaded,
+// solid or empty base, stored as they are, every image of one format whose
+// decode and encode return the same bytes; else 0.
+static int move_words(const StageDesc& d) {
+  if (d.post_end != d.post_begin + 1 || d.code[d.post_begin].op != OP_STORE) return 0;
+  const Slot& o = d.slot[d.code[d.post_begin].a];
+  if (o.fmt == FMT_GENERIC || o.width != d.width || o.height != d.height || d.height > 65535u * 16) return 0;
+  auto same = [&](const Slot& s) {
+    return s.fmt == o.fmt && s.bpp == o.bpp && s.width < (1u << 31) && s.height < (1u << 31);
+  };
+  const uint32_t nb = d.base_end - d.base_begin;
+  if (nb > 1) return 0;
+  if (nb == 1) {
+    const Instr& b = d.code[d.base_begin];
+    if (b.op == OP_LOAD ? !same(d.slot[b.a]) : b.op != OP_SOLID) return 0;
+  }
+  for (uint32_t l = 0; l < d.n_layers; ++l) {
+    const Layer& L = d.layer[l];
+    if (L.mode != LAYER_NEAREST_REPLACE || L.prog_end != L.prog_begin + 1) return 0;
+    if (L.inv[6] != 0.0 || L.inv[7] != 0.0 || L.inv[8] != 1.0) return 0;
+    const Instr& c = d.code[L.prog_begin];
+    if (c.op != OP_LOAD || !same(d.slot[c.a])) return 0;
+  }
+  return d.n_layers ? (int)(o.bpp / 4) : 0;
+}
+
 // Shape of the kernels of zh_field.hip a 2-D pointwise program has, its decode
 // table set; -1 for any other program.
 static int field_shape(StageDesc& d) {
@@ -1788,6 +1815,7 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
     // 64 x 16 tiles; the interpreter kernels stay valid on the same tiles as
     // the fallback for images the warp kernel cannot address.
     sp.desc.variant = bil ? warp_variant(sp.desc, flags) : -1;
+    if (!bil) sp.move = move_words(sp.desc);
     if (sp.desc.variant >= 0) {
       max_box = 0;
       choose_tiles({{64, 16}});
@@ -1817,6 +1845,8 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
            << "]";
       else if (sp.desc.variant >= 0)
         t2 << " [kernel " << zh_warp_name(sp.desc.variant) << lds << "]";
+      else if (sp.move)
+        t2 << " [move kernel]";
       sp.text = t2.str();
     }
     plan.stages.push_back(sp);

@@ -27,6 +27,7 @@ hipError_t zh_launch_any(uint32_t shape, const zh::StageDesc* d_dev, uint32_t wi
                          uint32_t cus, hipStream_t stream);
 hipError_t zh_launch_field(uint32_t shape, const zh::StageDesc* d_dev, uint32_t width, uint32_t height, uint32_t cus,
                            hipStream_t stream);
+hipError_t zh_launch_move(int words, const zh::StageDesc* d_dev, uint32_t width, uint32_t height, hipStream_t stream);
 hipError_t zh_launch_spec(int index, const zh::StageDesc* d_dev, uint32_t width, uint32_t height,
                           uint32_t cus, hipStream_t stream);
 hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, uint32_t cus,
@@ -931,7 +932,7 @@ zh_status zh_program_set_knob(zh_program* p, int32_t knob, const void* data, uin
     const StagePlan& b = p->plan.stages[i];
     same = a.desc.kind == b.desc.kind && a.tile_mode == b.tile_mode && a.desc.tiles_x == b.desc.tiles_x &&
            a.desc.tiles_y == b.desc.tiles_y && a.slot_ref == b.slot_ref && a.lds_bytes <= b.lds_bytes &&
-           a.spec == b.spec && a.jit == b.jit && a.any == b.any && a.field == b.field && a.fast == b.fast && a.desc.flat == b.desc.flat &&
+           a.spec == b.spec && a.jit == b.jit && a.any == b.any && a.field == b.field && a.move == b.move && a.fast == b.fast && a.desc.flat == b.desc.flat &&
            a.desc.variant == b.desc.variant && a.staged == b.staged;
   }
   p->params = params;
@@ -1054,6 +1055,11 @@ static zh_status bind(zh_program* p, const zh_binding* b, uint32_t n) {
         for (size_t k = 0; k < refs.size(); ++k)
           ok = ok && d.slot[k].ptr % d.slot[k].bpp == 0 && d.slot[k].row_stride % d.slot[k].bpp == 0;
         variant[s] = ok ? 3 : 0;
+      }
+      if (d.kind == STAGE_RESAMPLE && plan.stages[s].move) {
+        bool ok = true;
+        for (size_t k = 0; k < refs.size(); ++k) ok = ok && d.slot[k].ptr % 4 == 0 && d.slot[k].row_stride % 4 == 0;
+        variant[s] = ok ? 9 : 0;
       }
       if (d.kind == STAGE_POINTWISE && p->use_surrogates && s < p->d_surrogate.size() && p->d_surrogate[s] &&
           (p->surrogate_ok[s] || p->use_surrogates == 2)) {
@@ -1221,6 +1227,8 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
       } else if (first < p->variant.size() && p->variant[first] == 3) {
         ZH_HIP(zh_launch_warp(sp.desc.variant, sp.staged, d, sp.desc.tiles_x * sp.desc.tiles_y, (uint32_t)p->ctx->cus,
                               u.blocks_per_cu, s));
+      } else if (first < p->variant.size() && p->variant[first] == 9) {
+        ZH_HIP(zh_launch_move(sp.move, d, sp.desc.width, sp.desc.height, s));
       } else {
         ZH_HIP(zh_launch_resample(d, sp.tile_mode, sp.desc.tiles_x, sp.desc.tiles_y, sp.lds_bytes, s));
       }
