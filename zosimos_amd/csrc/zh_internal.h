@@ -196,7 +196,7 @@ struct Unit {
   uint32_t* d_prefix = nullptr;
   uint32_t grid = 0, lds = 0;
   uint32_t total_tiles = 0;
-  uint32_t blocks_per_cu = 0;    // persistent warp grids: 0 = as many as are resident
+  uint32_t blocks_per_cu = 0;    // warp grids: 0 = runs of tiles, else a persistent grid of so many
   uint32_t strip_w = 0;          // warp units: tiles dealt in strips this many tiles wide (0: by rows)
 };
 

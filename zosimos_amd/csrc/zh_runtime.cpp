@@ -32,6 +32,8 @@ hipError_t zh_launch_spec(int index, const zh::StageDesc* d_dev, uint32_t width,
                           uint32_t cus, hipStream_t stream);
 hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, uint32_t cus,
                                 hipStream_t stream);
+void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int staged, uint32_t* blocks,
+                  uint32_t* run);
 hipError_t zh_launch_warp(int index, int staged, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
                           uint32_t per_cu, hipStream_t stream);
 hipError_t zh_launch_warp_batch(int index, int staged, const zh::BatchDesc* b_dev, uint32_t total_tiles,
@@ -461,12 +463,12 @@ static void make_units(zh_program* p) {
   }
 }
 
-// The kernels' per-tile layer test (warp_tile in zh_warp.hip) on the host:
-// does any bilinear tap of the tile's pixel centres land in the layer's
-// source?  Widened by 1e-6 texel so that rounding never drops a tile the
-// kernel's own test would keep (a kept tile whose taps all miss adds 0).
-static bool tile_meets_layer(const Layer& L, double ex0, double ey0, double ex1, double ey1) {
-  if (L.covers_all) return true;
+// The kernels' per-tile layer tests (warp_tile in zh_warp_kernels.h) on the
+// host.  Bit 0: does any bilinear tap of the tile's pixel centres land in the
+// layer's source?  Widened by 1e-6 texel so that rounding never drops a tile
+// the kernel's own test would keep (a kept tile whose taps all miss adds 0).
+// Bit 8: do all of them, by as much (the lanes' fixed-point maps err by 1e-9)?
+static uint32_t tile_meets_layer(const Layer& L, double ex0, double ey0, double ex1, double ey1) {
   const double* m = L.inv;
   const double u[4] = {m[0] * ex0 + m[1] * ey0 + m[2], m[0] * ex1 + m[1] * ey0 + m[2], m[0] * ex0 + m[1] * ey1 + m[2],
                        m[0] * ex1 + m[1] * ey1 + m[2]};
@@ -476,8 +478,10 @@ static bool tile_meets_layer(const Layer& L, double ex0, double ey0, double ex1,
   const double umax = std::max(std::max(u[0], u[1]), std::max(u[2], u[3])) - 0.5;
   const double vmin = std::min(std::min(v[0], v[1]), std::min(v[2], v[3])) - 0.5;
   const double vmax = std::max(std::max(v[0], v[1]), std::max(v[2], v[3])) - 0.5;
-  const double e = 1e-6;
-  return umax > -1.0 - e && vmax > -1.0 - e && umin < (double)L.src_w + e && vmin < (double)L.src_h + e;
+  const double e = 1e-6, w = (double)L.src_w, h = (double)L.src_h;
+  const bool meets = L.covers_all || (umax > -1.0 - e && vmax > -1.0 - e && umin < w + e && vmin < h + e);
+  const bool inside = umin > e && vmin > e && umax < w - 1.0 - e && vmax < h - 1.0 - e;
+  return (meets ? 1u : 0u) | (meets && inside ? 256u : 0u);
 }
 
 // The tile-layer masks of warp stage s for its current tile shape (host
@@ -489,7 +493,7 @@ static zh_status tile_layer_masks(zh_program* p, size_t s) {
     p->d_tile_layers.resize(p->plan.stages.size(), nullptr);
     p->tile_layer_words.resize(p->plan.stages.size(), 0);
   }
-  const uint32_t tiles = d.tiles_x * d.tiles_y, words = (tiles + 3) / 4;
+  const uint32_t tiles = d.tiles_x * d.tiles_y, words = (tiles + 1) / 2;
   std::vector<uint32_t> m(std::max(1u, words), 0u);
   const int TW = (int)d.tile_w, TH = (int)d.tile_h, W = (int)d.width, H = (int)d.height;
   for (uint32_t ty = 0; ty < d.tiles_y; ++ty)
@@ -497,10 +501,11 @@ static zh_status tile_layer_masks(zh_program* p, size_t s) {
       const double ex0 = (double)tx * TW + 0.5, ey0 = (double)ty * TH + 0.5;
       const double ex1 = std::min((int)tx * TW + TW, W) - 0.5, ey1 = std::min((int)ty * TH + TH, H) - 0.5;
       uint32_t bits = 0;
-      for (uint32_t l = 0; l < d.n_layers; ++l)
-        if (tile_meets_layer(d.layer[l], ex0, ey0, ex1, ey1)) bits |= 1u << l;
+      for (uint32_t l = 0; l < d.n_layers; ++l) bits |= tile_meets_layer(d.layer[l], ex0, ey0, ex1, ey1) << l;
+      // Only whole tiles take the path without tests.
+      if ((int)(tx + 1) * TW > W || (int)(ty + 1) * TH > H) bits &= 255u;
       const uint32_t t = ty * d.tiles_x + tx;
-      m[t >> 2] |= bits << ((t & 3u) * 8u);
+      m[t >> 1] |= bits << ((t & 1u) * 16u);
     }
   if (p->h_tile_layers.size() < p->plan.stages.size()) p->h_tile_layers.resize(p->plan.stages.size());
   if (p->d_tile_layers[s] && p->h_tile_layers[s] == m) {
@@ -1155,12 +1160,13 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
     }
     if (all_warp) {
       if (p->plan.stages[u.ids[0]].desc.variant >= kJitWarpBase) {
-        const uint32_t first = u.ids[0], res = p->jit_batch_resident[first];
-        const uint32_t bpc = u.blocks_per_cu ? std::min(u.blocks_per_cu, res) : res;
-        const uint32_t blocks = std::min<uint32_t>(u.total_tiles, bpc * (uint32_t)p->ctx->cus);
+        const uint32_t first = u.ids[0];
+        uint32_t blocks, run;
+        zh_warp_grid(u.total_tiles, p->jit_batch_resident[first], (uint32_t)p->ctx->cus, u.blocks_per_cu, u.staged,
+                     &blocks, &run);
         if (blocks == 0) return ZH_OK;
         const BatchDesc* bd = u.d_batch;
-        void* args[] = {&bd};
+        void* args[] = {&bd, &run};
         ZH_HIP(hipModuleLaunchKernel(p->jit_batch_fn[first], blocks, 1, 1, kBlock, 1, 1, 0, s, args, nullptr));
         return ZH_OK;
       }
@@ -1216,13 +1222,13 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
     }
     case STAGE_RESAMPLE:
       if (first < p->variant.size() && p->variant[first] == 3 && sp.desc.variant >= kJitWarpBase) {
-        // A run-time warp form: the persistent grid of zh_launch_warp.
-        const uint32_t res = p->jit_resident[first];
-        const uint32_t bpc = u.blocks_per_cu ? std::min(u.blocks_per_cu, res) : res;
-        const uint32_t blocks = std::min<uint32_t>(sp.desc.tiles_x * sp.desc.tiles_y, bpc * (uint32_t)p->ctx->cus);
+        // A run-time warp form: the grid of zh_launch_warp.
+        uint32_t blocks, run;
+        zh_warp_grid(sp.desc.tiles_x * sp.desc.tiles_y, p->jit_resident[first], (uint32_t)p->ctx->cus, u.blocks_per_cu,
+                     sp.staged, &blocks, &run);
         if (blocks == 0) break;
         const StageDesc* dp = d;
-        void* args[] = {&dp};
+        void* args[] = {&dp, &run};
         ZH_HIP(hipModuleLaunchKernel(p->jit_stage_fn[first], blocks, 1, 1, kBlock, 1, 1, 0, s, args, nullptr));
       } else if (first < p->variant.size() && p->variant[first] == 3) {
         ZH_HIP(zh_launch_warp(sp.desc.variant, sp.staged, d, sp.desc.tiles_x * sp.desc.tiles_y, (uint32_t)p->ctx->cus,

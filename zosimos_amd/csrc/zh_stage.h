@@ -215,8 +215,8 @@ struct StageDesc {
   uint32_t copy_rows, copy_pad;
   const void* srgb_lut;       // the context's 8-bit sRGB tables (Luts of zh_codec.h)
   // Warp stages: per tile (row-major) a byte of the layers whose footprint
-  // meets the tile, four tiles per word (bit l: layer l); null: the kernel
-  // tests each layer itself.
+  // meets the tile and a byte of those whose source holds every tap of it, two
+  // tiles per word (bit l: layer l); null: the kernel tests each layer itself.
   const uint32_t* tile_layers;
   TableDesc table[2];         // any-format kernels: the decode tables of their loads
   uint32_t* error_flag;       // set to 1 by a kernel that met an impossible case

@@ -7,10 +7,11 @@
 // registered forms (zh_spec.h) run here as straight-line code:
 //
 //   * the output is cut into tiles of tile_w x tile_h pixels (one workgroup
-//     of 256 lanes, kPix = 4 horizontally adjacent pixels per lane); a
-//     persistent grid walks the tiles with a stride;
+//     of 256 lanes, kPix = 4 horizontally adjacent pixels per lane); each
+//     workgroup takes a short run of tiles (deal_tiles);
 //   * per tile and layer, the layer is skipped when it misses the tile (the
-//     host's per-tile mask, or the tile's footprint mapped in FP64); each
+//     host's per-tile mask, or the tile's footprint mapped in FP64), and its
+//     border tests are when the host found every tap inside its source; each
 //     lane's first pixel centre and the step between the lane's pixels are
 //     held in 32.32 fixed point, computed with integers from the layer's map
 //     in fixed point (the tile's part uniform), so every pixel's map is one
@@ -135,6 +136,12 @@ __device__ __forceinline__ bool layer_hits(const Layer& L, double ex0, double ey
   return umax > -1.0 && vmax > -1.0 && umin < (double)L.src_w && vmin < (double)L.src_h;
 }
 
+// The tile's word of the host's masks: bits 0-7 the layers that meet it, bits
+// 8-15 those whose source holds every tap of its pixels.
+__device__ __forceinline__ uint32_t tile_masks(const uint32_t* tl, uint32_t t) {
+  return (cword(tl, t >> 1) >> ((t & 1u) * 16u)) & 0xffffu;
+}
+
 // layer_hits over the pixel-centre extent of tile (tx, ty) (clipped to the
 // image).  The fallback for stages without the host's per-tile masks; kept
 // out of line so that its FP64 set-up is not hoisted onto every tile's path.
@@ -222,38 +229,76 @@ __device__ __forceinline__ typename RawT<F>::type pair_half(const typename PairT
   }
 }
 
+// 'Over' X the bilinear sample of four taps (c1: the upper source's) with
+// weights w.
+template <class V>
+__device__ __forceinline__ void blend_taps(const LayerArgs& a, const typename RawT<V::F>::type* c0,
+                                           const typename RawT<V::F>::type* c1, const float* w, float4& X,
+                                           const Luts* L) {
+  constexpr bool A8 = fmt_bpp(V::F) == 4 && V::SRC == WSRC_ONE;
+  float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const float4 c = raw_dec<V::F>(c0[t], L);
+    if constexpr (V::SRC == WSRC_OVER2) {
+      // Premultiplied 'over' of the two sources, then weighted.
+      const float4 lo = premul4(c);
+      const float4 h = premul4(raw_dec<V::F>(c1[t], L));
+      const float q = 1.0f - h.w, wt = w[t];
+      const float4 m = make_float4(fmaf(lo.x, q, h.x), fmaf(lo.y, q, h.y), fmaf(lo.z, q, h.z), fmaf(lo.w, q, h.w));
+      s = make_float4(fmaf(m.x, wt, s.x), fmaf(m.y, wt, s.y), fmaf(m.z, wt, s.z), fmaf(m.w, wt, s.w));
+    } else {
+      float al = c.w;
+      if constexpr (A8) al = (float)(c0[t] >> 24);
+      // Half alphas: w * a as fma(a, w, +0), which compiles to one mixed-
+      // precision fma reading the f16 half directly (the same value but
+      // for the sign of a zero product).
+      const float wa = V::F == FMT_F16 ? __builtin_fmaf(al, w[t], 0.0f) : w[t] * al;
+      s = make_float4(fmaf(c.x, wa, s.x), fmaf(c.y, wa, s.y), fmaf(c.z, wa, s.z), s.w + wa);
+    }
+  }
+  if constexpr (V::MAT) {
+    const float r = a.m[0] * s.x + a.m[1] * s.y + a.m[2] * s.z;
+    const float g = a.m[3] * s.x + a.m[4] * s.y + a.m[5] * s.z;
+    const float b = a.m[6] * s.x + a.m[7] * s.y + a.m[8] * s.z;
+    s = make_float4(r, g, b, s.w);
+  }
+  const float kk = 1.0f - s.w;
+  X = make_float4(fmaf(X.x, kk, s.x), fmaf(X.y, kk, s.y), fmaf(X.z, kk, s.z), fmaf(X.w, kk, s.w));
+}
+
+// Byte offsets and weights of a lane's taps: off[k][r] the tap pair of row r (or,
+// for 16-byte texels, off[k][t] tap t), w[k][t] tap t's weight.  Returns false
+// when no tap of the lane lies in the source.
 template <class V, bool SEP>
-__device__ __forceinline__ void layer_taps(const LayerArgs& a, const LaneMap& mp, int n, Px& X, const Luts* L) {
-  typedef typename RawT<V::F>::type R;
+__device__ __forceinline__ bool tap_weights(const LayerArgs& a, const LaneMap& mp, int n, uint32_t (*off)[4],
+                                            float (*w)[4]) {
   constexpr uint32_t B = fmt_bpp(V::F);
   // 4- and 8-byte texels: the two taps of a row are one load.  The left tap
   // is clamped to [0, sw - 2] (the planner admits sources at least 2 texels
   // wide), so the pair lies inside its row, and each texel of the pair gets
-  // the tent weight max(0, 1 - |sample - texel|): the bilinear weight for
-  // the sample's own taps, 0 for a texel the clamp substituted at a border.
+  // the tent weight max(0, 1 - |sample - texel|): the bilinear weight for the
+  // sample's own taps, 0 for a texel the clamp substituted at a border.
   constexpr bool PAIR = B <= 8;
-  typedef typename PairT<B <= 8 ? B : 8>::type PR;
   // One-source 8-bit formats weigh each tap by its alpha byte: the 1/255 of
   // the byte's value goes into the row weights instead of every tap.
-  constexpr bool A8 = B == 4 && V::SRC == WSRC_ONE;
-  constexpr float kA = A8 ? 1.0f / 255.0f : 1.0f;
-  uint32_t off[kPix][4];
-  float w[kPix][4];
+  constexpr float kA = B == 4 && V::SRC == WSRC_ONE ? 1.0f / 255.0f : 1.0f;
   bool any = false;
   // Rows: shared by the lane's pixels when the map is separable.
-  float wy0s = 0.0f, wy1s = 0.0f;
-  uint32_t r0s = 0, r1s = 0;
-  bool yas = false, ybs = false;
-  if constexpr (SEP) {
-    const int j = fx_int(mp.v0);
-    const float ay = fx_frac(mp.v0);
-    yas = (unsigned)j < (unsigned)a.sh;
-    ybs = (unsigned)(j + 1) < (unsigned)a.sh;
-    wy0s = yas ? (1.0f - ay) * kA : 0.0f;
-    wy1s = ybs ? ay * kA : 0.0f;
-    r0s = (uint32_t)__mul24(j, (int)a.stride);
-    r1s = r0s + a.stride;
-  }
+  float wy0 = 0.0f, wy1 = 0.0f;
+  uint32_t r0 = 0, r1 = 0;
+  bool ya = false, yb = false;
+  auto rows = [&](int64_t v) {
+    const int j = fx_int(v);
+    const float ay = fx_frac(v);
+    ya = (unsigned)j < (unsigned)a.sh;
+    yb = (unsigned)(j + 1) < (unsigned)a.sh;
+    wy0 = ya ? (1.0f - ay) * kA : 0.0f;
+    wy1 = yb ? ay * kA : 0.0f;
+    r0 = (uint32_t)__mul24(j, (int)a.stride);
+    r1 = r0 + a.stride;
+  };
+  if constexpr (SEP) rows(mp.v0);
 #pragma unroll
   for (int k = 0; k < kPix; ++k) {
     const int64_t uk = mp.u0 + mp.su * k;
@@ -261,27 +306,7 @@ __device__ __forceinline__ void layer_taps(const LayerArgs& a, const LaneMap& mp
     const float ax = fx_frac(uk);
     const bool in = k < n;
     const bool xa = in && (unsigned)i < (unsigned)a.sw, xb = in && (unsigned)(i + 1) < (unsigned)a.sw;
-    bool ya, yb;
-    float wy0, wy1;
-    uint32_t r0, r1;
-    if constexpr (SEP) {
-      ya = yas;
-      yb = ybs;
-      wy0 = wy0s;
-      wy1 = wy1s;
-      r0 = r0s;
-      r1 = r1s;
-    } else {
-      const int64_t vk = mp.v0 + mp.sv * k;
-      const int j = fx_int(vk);
-      const float ay = fx_frac(vk);
-      ya = (unsigned)j < (unsigned)a.sh;
-      yb = (unsigned)(j + 1) < (unsigned)a.sh;
-      wy0 = ya ? (1.0f - ay) * kA : 0.0f;
-      wy1 = yb ? ay * kA : 0.0f;
-      r0 = (uint32_t)__mul24(j, (int)a.stride);
-      r1 = r0 + a.stride;
-    }
+    if constexpr (!SEP) rows(mp.v0 + mp.sv * k);
     any = any || ((xa || xb) && (ya || yb));
     if constexpr (PAIR) {
       const int ic = min(max(i, 0), a.sw - 2);
@@ -308,7 +333,64 @@ __device__ __forceinline__ void layer_taps(const LayerArgs& a, const LaneMap& mp
       off[k][3] = opaque(off[k][2] + B);
     }
   }
-  if (!any) return;
+  return any;
+}
+
+// The same for a tile whose every pixel exists and whose every tap lies inside
+// the source (the host's mask): nothing is clamped, masked or tested, about 20
+// of the 55 vector instructions a pixel and layer.  The weights are
+// tap_weights' values bit for bit: for a sample between texels i and i + 1 the
+// tent weights are 1 - f and 1 - (1 - f), and the row weights are unmasked.
+template <class V, bool SEP>
+__device__ __forceinline__ void tap_weights_inside(const LayerArgs& a, const LaneMap& mp, uint32_t (*off)[4],
+                                                   float (*w)[4]) {
+  constexpr uint32_t B = fmt_bpp(V::F);
+  constexpr bool PAIR = B <= 8;
+  constexpr float kA = B == 4 && V::SRC == WSRC_ONE ? 1.0f / 255.0f : 1.0f;
+  float wy0 = 0.0f, wy1 = 0.0f;
+  uint32_t row = 0;
+  auto rows = [&](int64_t v) {
+    const float ay = fx_frac(v);
+    wy0 = (1.0f - ay) * kA;
+    wy1 = ay * kA;
+    row = __umul24((uint32_t)fx_int(v), a.stride);
+  };
+  if constexpr (SEP) rows(mp.v0);
+#pragma unroll
+  for (int k = 0; k < kPix; ++k) {
+    const int64_t uk = mp.u0 + mp.su * k;
+    if constexpr (!SEP) rows(mp.v0 + mp.sv * k);
+    const float ax = fx_frac(uk), wl = 1.0f - ax, wh = PAIR ? 1.0f - wl : ax;
+    w[k][0] = wl * wy0;
+    w[k][1] = wh * wy0;
+    w[k][2] = wl * wy1;
+    w[k][3] = wh * wy1;
+    const uint32_t at = row + (uint32_t)fx_int(uk) * B;
+    if constexpr (PAIR) {
+      off[k][0] = at;
+      off[k][1] = at + a.stride;
+    } else {
+      off[k][0] = at;
+      off[k][1] = at + B;
+      off[k][2] = at + a.stride;
+      off[k][3] = at + a.stride + B;
+    }
+  }
+}
+
+template <class V, bool SEP>
+__device__ __forceinline__ void layer_taps(const LayerArgs& a, const LaneMap& mp, bool inside, int n, Px& X,
+                                           const Luts* L) {
+  typedef typename RawT<V::F>::type R;
+  constexpr uint32_t B = fmt_bpp(V::F);
+  constexpr bool PAIR = B <= 8;
+  typedef typename PairT<B <= 8 ? B : 8>::type PR;
+  uint32_t off[kPix][4];
+  float w[kPix][4];
+  if (inside)  // uniform
+    tap_weights_inside<V, SEP>(a, mp, off, w);
+  else if (!tap_weights<V, SEP>(a, mp, n, off, w))
+    return;
   R t0[kPix][4], t1[kPix][4];
   PR p0[kPix][2], p1[kPix][2];
   if constexpr (PAIR) {
@@ -333,35 +415,18 @@ __device__ __forceinline__ void layer_taps(const LayerArgs& a, const LaneMap& mp
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int k = 0; k < kPix; ++k) {
-    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    R c0[4], c1[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const float4 c = raw_dec<V::F>(PAIR ? pair_half<V::F>(p0[k][t >> 1], t & 1) : t0[k][t], L);
-      if constexpr (V::SRC == WSRC_OVER2) {
-        // Premultiplied 'over' of the two sources, then weighted.
-        const float4 lo = premul4(c);
-        const float4 h = premul4(raw_dec<V::F>(PAIR ? pair_half<V::F>(p1[k][t >> 1], t & 1) : t1[k][t], L));
-        const float q = 1.0f - h.w, wt = w[k][t];
-        const float4 m = make_float4(fmaf(lo.x, q, h.x), fmaf(lo.y, q, h.y), fmaf(lo.z, q, h.z), fmaf(lo.w, q, h.w));
-        s = make_float4(fmaf(m.x, wt, s.x), fmaf(m.y, wt, s.y), fmaf(m.z, wt, s.z), fmaf(m.w, wt, s.w));
+      if constexpr (PAIR) {
+        c0[t] = pair_half<V::F>(p0[k][t >> 1], t & 1);
+        if constexpr (V::SRC == WSRC_OVER2) c1[t] = pair_half<V::F>(p1[k][t >> 1], t & 1);
       } else {
-        float al = c.w;
-        if constexpr (A8) al = (float)((PAIR ? pair_half<V::F>(p0[k][t >> 1], t & 1) : t0[k][t]) >> 24);
-        // Half alphas: w * a as fma(a, w, +0), which compiles to one mixed-
-        // precision fma reading the f16 half directly (the same value but
-        // for the sign of a zero product).
-        const float wa = V::F == FMT_F16 ? __builtin_fmaf(al, w[k][t], 0.0f) : w[k][t] * al;
-        s = make_float4(fmaf(c.x, wa, s.x), fmaf(c.y, wa, s.y), fmaf(c.z, wa, s.z), s.w + wa);
+        c0[t] = t0[k][t];
+        if constexpr (V::SRC == WSRC_OVER2) c1[t] = t1[k][t];
       }
     }
-    if constexpr (V::MAT) {
-      const float r = a.m[0] * s.x + a.m[1] * s.y + a.m[2] * s.z;
-      const float g = a.m[3] * s.x + a.m[4] * s.y + a.m[5] * s.z;
-      const float b = a.m[6] * s.x + a.m[7] * s.y + a.m[8] * s.z;
-      s = make_float4(r, g, b, s.w);
-    }
-    const float kk = 1.0f - s.w;
-    X[k] = make_float4(fmaf(X[k].x, kk, s.x), fmaf(X[k].y, kk, s.y), fmaf(X[k].z, kk, s.z), fmaf(X[k].w, kk, s.w));
+    blend_taps<V>(a, c0, c1, w[k], X[k], L);
   }
 }
 
@@ -398,7 +463,7 @@ __device__ __forceinline__ void warp_tile(CDesc d, uint32_t tx, uint32_t ty, con
   // Layers meeting this tile: the host's per-tile mask when there is one.
   const uint32_t* tl = d->tile_layers;
   const uint32_t t = ty * d->tiles_x + tx;
-  const uint32_t lmask = tl ? (cword(tl, t >> 2) >> ((t & 3u) * 8u)) & 255u : 255u;
+  const uint32_t lmask = tl ? tile_masks(tl, t) : 255u;
   for (uint32_t l = 0; l < nl; ++l) {
     if (!((lmask >> l) & 1u)) continue;  // uniform
     const Layer Ly = ldc(&d->layer[l]);
@@ -409,7 +474,7 @@ __device__ __forceinline__ void warp_tile(CDesc d, uint32_t tx, uint32_t ty, con
     // SEP variant only when every layer has one) are separable: the lane's
     // pixels share one source row pair, computed once.
     const LaneMap mp = lane_map<V::SEP>(Ly, tx * (uint32_t)TW, ty * (uint32_t)TH, lx, ly, lanes_x);
-    layer_taps<V, V::SEP>(a, mp, n, X, L);
+    layer_taps<V, V::SEP>(a, mp, ((lmask >> (8 + l)) & 1u) != 0, n, X, L);
   }
 
   if (n == 0) return;
@@ -538,7 +603,7 @@ __device__ __forceinline__ BoxTile box_tile(CDesc d, uint32_t tx, uint32_t ty) {
   const uint32_t* tl = d->tile_layers;
   const uint32_t t = ty * d->tiles_x + tx;
   if (tl) {
-    s.hit = (cword(tl, t >> 2) >> ((t & 3u) * 8u)) & 1u;
+    s.hit = tile_masks(tl, t) & 1u;
   } else {
     const int W = (int)d->width, H = (int)d->height;
     const double ex1 = min((int)tx * TW + TW, W) - 0.5, ey1 = min((int)ty * TH + TH, H) - 0.5;
@@ -777,46 +842,64 @@ __device__ __forceinline__ void warp_staged_batch(const BatchDesc* bb) {
               raw, box, &luts);
 }
 
+// Tiles a workgroup takes.  run = 0: a persistent grid, each workgroup taking
+// every gridDim-th tile.  run > 0: run consecutive tiles, so that the hardware
+// dispatcher balances the load: the waves of a SIMD do not progress evenly
+// (the older ones win arbitration), and equal shares of a persistent grid end
+// at 50-100% of its time, the last third of it at falling occupancy.
+struct Deal {
+  uint32_t first, step, end;
+};
+__device__ __forceinline__ Deal deal_tiles(uint32_t total, uint32_t run) {
+  if (run == 0) return Deal{virtual_block(), gridDim.x, total};
+  // Blocks go round-robin to the 8 XCDs; each XCD takes kRuns neighbouring runs
+  // of every 8 kRuns, so the tiles it works on at once share their halo texels
+  // in its L2.
+  constexpr uint32_t kRuns = 64;
+  const uint32_t b = blockIdx.x, round = b / (8u * kRuns), full = gridDim.x / (8u * kRuns);
+  const uint32_t v = round < full ? round * 8u * kRuns + (b % 8u) * kRuns + (b / 8u) % kRuns : b;
+  return Deal{v * run, 1u, min(v * run + run, total)};
+}
+
 template <class V>
-__device__ __forceinline__ void warp_stage(const StageDesc* dd) {
+__device__ __forceinline__ void warp_stage(const StageDesc* dd, uint32_t run) {
   const CDesc d = as_const(dd);
   __shared__ Luts luts;
   if constexpr (needs_lut<V>()) {
     load_lut(d, &luts);
     __syncthreads();
   }
-  const uint32_t tiles = d->tiles_x * d->tiles_y;
-  for (uint32_t t = virtual_block(); t < tiles; t += gridDim.x) {
+  const Deal q = deal_tiles(d->tiles_x * d->tiles_y, run);
+  for (uint32_t t = q.first; t < q.end; t += q.step) {
     uint32_t tx, ty;
     tile_xy(d, t, tx, ty);
     warp_tile<V>(d, tx, ty, &luts);
   }
 }
 
-// Persistent grid over the tiles of a batch of stages of one form (images of
-// uneven sizes): tile j belongs to the last stage s with prefix[s] <= j.  The
-// tiles are dealt exactly as one stage's tiles are (grid-stride, XCD-aware),
-// so at any moment the grid works on one contiguous band of tiles and their
-// source rows stay in the L2 and the TLBs.  A workgroup's tiles only move
-// forward, so after one binary search its stage is found by walking the
-// prefix, less than one scalar load per tile on average.
+// The tiles of a batch of stages of one form (images of uneven sizes): tile j
+// belongs to the last stage s with prefix[s] <= j.  The tiles are dealt
+// exactly as one stage's tiles are, so at any moment the grid works on one
+// contiguous band of tiles and their source rows stay in the L2 and the TLBs.
+// A workgroup's tiles only move forward, so after one binary search its stage
+// is found by walking the prefix, less than one scalar load per tile on
+// average.
 template <class V>
-__device__ __forceinline__ void warp_batch(const BatchDesc* bb) {
+__device__ __forceinline__ void warp_batch(const BatchDesc* bb, uint32_t run) {
   const CBatch b = (CBatch)(uintptr_t)bb;
   __shared__ Luts luts;
   if constexpr (needs_lut<V>()) {
     load_lut(as_const(b->stages), &luts);
     __syncthreads();
   }
-  const uint32_t total = b->total_tiles;
-  const uint32_t j0 = virtual_block();
-  if (j0 >= total) return;
+  const Deal q = deal_tiles(b->total_tiles, run);
+  if (q.first >= q.end) return;
   uint32_t lo = 0, hi = b->n_stages;
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) / 2;
-    if (cword(b->tile_prefix, mid) <= j0) lo = mid; else hi = mid;
+    if (cword(b->tile_prefix, mid) <= q.first) lo = mid; else hi = mid;
   }
-  for (uint32_t j = j0; j < total; j += gridDim.x) {
+  for (uint32_t j = q.first; j < q.end; j += q.step) {
     while (cword(b->tile_prefix, lo + 1) <= j) ++lo;  // uniform
     const CDesc d = as_const(b->stages + cword(b->stage_ids, lo));
     uint32_t tx, ty;
