@@ -30,8 +30,7 @@ hipError_t zh_launch_field(uint32_t shape, const zh::StageDesc* d_dev, uint32_t 
 hipError_t zh_launch_move(int words, const zh::StageDesc* d_dev, uint32_t width, uint32_t height, hipStream_t stream);
 hipError_t zh_launch_spec(int index, const zh::StageDesc* d_dev, uint32_t width, uint32_t height,
                           uint32_t cus, hipStream_t stream);
-hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, uint32_t cus,
-                                hipStream_t stream);
+hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, hipStream_t stream);
 void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int staged, uint32_t* blocks,
                   uint32_t* run);
 hipError_t zh_launch_warp(int index, int staged, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
@@ -546,9 +545,15 @@ static zh_status upload_buffers(zh_program* p) {
 static zh_status alloc_batch(zh_program* p, const uint32_t* ids, size_t n, bool spec, uint32_t* counter,
                              BatchDesc** d_batch, uint32_t** d_prefix, uint32_t** d_ids, uint32_t* total) {
   std::vector<uint32_t> prefix(n + 1, 0);
+  auto pixels = [&](size_t k) {
+    return (uint64_t)p->plan.stages[ids[k]].desc.width * p->plan.stages[ids[k]].desc.height;
+  };
+  uint64_t all = 0;
+  for (size_t k = 0; k < n; ++k) all += pixels(k);
+  const uint32_t steps = spec_steps(all, (uint32_t)p->ctx->cus);
   for (size_t k = 0; k < n; ++k) {
     const StageDesc& d = p->plan.stages[ids[k]].desc;
-    const uint64_t chunks = ((uint64_t)d.width * d.height + kSpecChunkPixels - 1) / kSpecChunkPixels;
+    const uint64_t chunk = (uint64_t)kBlock * kPix * steps, chunks = (pixels(k) + chunk - 1) / chunk;
     prefix[k + 1] = prefix[k] + (spec ? (uint32_t)chunks : d.tiles_x * d.tiles_y);
   }
   ZH_ALLOC(p, sizeof(BatchDesc), d_batch);
@@ -559,6 +564,7 @@ static zh_status alloc_batch(zh_program* p, const uint32_t* ids, size_t n, bool 
   BatchDesc b{};
   b.n_stages = (uint32_t)n;
   b.total_tiles = prefix.back();
+  b.chunk_groups = steps;
   b.counter = counter;
   b.stages = p->d_stages;
   b.stage_ids = *d_ids;
@@ -1133,16 +1139,15 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
       all_jit = all_jit && p->variant[id] == 6;
     }
     if (all_spec) {
-      ZH_HIP(zh_launch_spec_batch(p->plan.stages[u.ids[0]].spec, u.d_batch, u.total_tiles, (uint32_t)p->ctx->cus, s));
+      ZH_HIP(zh_launch_spec_batch(p->plan.stages[u.ids[0]].spec, u.d_batch, u.total_tiles, s));
       return ZH_OK;
     }
     if (all_jit) {
       const uint32_t first = u.ids[0];
-      const uint32_t blocks = std::min<uint32_t>(u.total_tiles, p->jit_batch_resident[first] * (uint32_t)p->ctx->cus);
-      if (blocks == 0) return ZH_OK;
+      if (u.total_tiles == 0) return ZH_OK;
       const BatchDesc* bd = u.d_batch;
       void* args[] = {&bd};
-      ZH_HIP(hipModuleLaunchKernel(p->jit_batch_fn[first], blocks, 1, 1, kBlock, 1, 1, 0, s, args, nullptr));
+      ZH_HIP(hipModuleLaunchKernel(p->jit_batch_fn[first], u.total_tiles, 1, 1, kBlock, 1, 1, 0, s, args, nullptr));
       return ZH_OK;
     }
     bool all_warp = u.warp;

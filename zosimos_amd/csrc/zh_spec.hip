@@ -83,16 +83,12 @@ hipError_t zh_launch_spec(int index, const zh::StageDesc* d_dev, uint32_t width,
   return hipGetLastError();
 }
 
-// A batch of stages of signature `index`: total_chunks chunks of
-// kSpecChunkPixels (the BatchDesc prefix counts chunks).
-hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, uint32_t cus,
-                                hipStream_t stream) {
+// A batch of stages of signature `index`: total_chunks chunks (the BatchDesc
+// prefix counts them), one workgroup each.
+hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, hipStream_t stream) {
   if (index < 0 || index >= zh::spec::kNumEntries) return hipErrorInvalidValue;
-  static uint32_t resident[zh::spec::kNumEntries] = {};
-  if (!resident[index]) resident[index] = zh::resident_blocks((const void*)zh::spec::kEntries[index].batch, 1);
-  const uint32_t blocks = std::min(total_chunks, resident[index] * cus);
-  if (blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL(zh::spec::kEntries[index].batch, dim3(blocks), dim3(zh::kBlock), 0, stream, b_dev);
+  if (total_chunks == 0) return hipSuccess;
+  hipLaunchKernelGGL(zh::spec::kEntries[index].batch, dim3(total_chunks), dim3(zh::kBlock), 0, stream, b_dev);
   return hipGetLastError();
 }
 

@@ -27,10 +27,17 @@ constexpr int kMaxInstr = 64;
 constexpr int kMaxParams = 256;  // floats
 constexpr int kMaxLayers = 8;
 constexpr int kBlock = 256;      // threads per workgroup
-// A batch of flat pointwise stages is dealt in chunks of kSpecChunkGroups
-// groups of kPix pixels per lane of one workgroup (16,384 pixels).
-constexpr uint32_t kSpecChunkGroups = 16;
-constexpr uint64_t kSpecChunkPixels = (uint64_t)kBlock * kPix * kSpecChunkGroups;
+// Steps (of kPix pixels per lane of a workgroup) in a chunk of a batch of flat
+// pointwise stages: up to 16, while that leaves 8 chunks per compute unit.
+// Always 16 leaves small batches on few compute units (2 images 276x270: 15.5
+// us against 7.2; 3 images 1000x600: 16.9 / 8.6); 4 and 8 repeat more set-up
+// in large ones (16 images 3840x2160: 251 and 245 us, 16 243, 32 246), and 2 or
+// 4 chunks per compute unit balance worse (14 images 1435x748: 36-37 us, 8 32).
+constexpr uint32_t spec_steps(uint64_t pixels, uint32_t cus) {
+  const uint64_t s = pixels / ((uint64_t)kBlock * kPix * 8 * (cus ? cus : 1));
+  return s < 1 ? 1u : s > 16 ? 16u : (uint32_t)s;
+}
+
 // LDS bytes available to one resample tile (float4 texels).
 constexpr int kTileLdsBytes = 64 * 1024;
 // Staged warp tiles: float4 texels of a tile's source box in LDS (25.6 KB;
@@ -230,6 +237,7 @@ struct StageDesc {
 struct BatchDesc {
   uint32_t n_stages;
   uint32_t total_tiles;
+  uint32_t chunk_groups;        // pointwise batches: steps of a chunk
   uint32_t* counter;            // reset by a one-lane kernel before each launch
   const StageDesc* stages;      // the program's descriptors
   const uint32_t* stage_ids;    // n_stages indices into `stages`
