@@ -23,7 +23,7 @@ def test_unregistered_chain_is_compiled_at_run_time():
 
 def test_registered_and_unsupported_chains():
     assert "[kernel c2_over" in describe(W.c2(64, 32).commands)
-    # SrLab2's non-linearity has no specialised body: the interpreter runs it
+    # SrLab2's encode is registered too
     d = z.Descriptor.rgba8_srgb(32, 32)
     cmd = z.CommandBuffer()
     i = cmd.input(d)

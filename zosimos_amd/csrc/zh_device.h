@@ -121,12 +121,25 @@ __device__ __forceinline__ float cbrt_s(float x) { return copysignf(pow_pos(fabs
 // SrLab2's cone non-linearity and its inverse (srlab2.frag:87-120).  The
 // shader's pow of a negative base is undefined; below -216/24389 the cube
 // root is taken with its sign.
+//
+// x / c for a constant c in 3 instructions for the general division's 11: the
+// product with 1/c, corrected by its exact remainder (Markstein).  Compared
+// over every float x, this is the rounded quotient for c = 24389, for 2700
+// where |x| > 4.8e-38 (a unit of 1.4e-45 off below) and for 1.16 where |x| >
+// 6.2e-32; v + 0.16 with |v| >= 0.08 is 0 or at least 7e-9.  Infinite x gives
+// NaN, so the last division takes the hardware's fix-up.
+__device__ __forceinline__ float div_const(float x, float c, float rc) {
+  const float q = x * rc;
+  return fmaf(fmaf(-q, c, x), rc, q);
+}
 __device__ __forceinline__ float srlab_nl(float v) {
-  return fabsf(v) < 216.0f / 24389.0f ? v * 24389.0f / 2700.0f : 1.16f * cbrt_s(v) - 0.16f;
+  return fabsf(v) < 216.0f / 24389.0f ? div_const(v * 24389.0f, 2700.0f, 1.0f / 2700.0f)
+                                      : fmaf(1.16f, cbrt_s(v), -0.16f);
 }
 __device__ __forceinline__ float srlab_nl_inv(float v) {
-  if (fabsf(v) < 0.08f) return v * 2700.0f / 24389.0f;
-  const float p = (v + 0.16f) / 1.16f;
+  if (fabsf(v) < 0.08f) return div_const(v * 2700.0f, 24389.0f, 1.0f / 24389.0f);
+  const float x = v + 0.16f;
+  const float p = __builtin_amdgcn_div_fixupf(div_const(x, 1.16f, 1.0f / 1.16f), 1.16f, x);
   return p * p * p;
 }
 

@@ -221,7 +221,7 @@ bool jit_supported(const uint16_t* sig, int n) {
   for (int i = 0; i < n; ++i) {
     const uint32_t op = sig[i] & 0xffu;
     if (op != OP_LOAD && op != OP_STORE && op != OP_MAT3 && op != OP_CBRT && op != OP_CUBE && op != OP_CLAMP01 &&
-        op != OP_PREMUL && op != OP_UNPREMUL && op != OP_OVER)
+        op != OP_PREMUL && op != OP_UNPREMUL && op != OP_OVER && op != OP_SRLAB && op != OP_SRLAB_INV)
       return false;
   }
   return true;

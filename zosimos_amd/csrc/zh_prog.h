@@ -53,9 +53,18 @@ struct Prog {
     if (fmt_bpp(el_fmt(el[0])) != 4 || fmt_bpp(el_fmt(el[n - 1])) != 4) return false;
     for (int k = 1; k < n - 1; ++k) {
       const uint32_t o = el_op(el[k]);
-      if (o != OP_MAT3 && o != OP_CBRT && o != OP_CUBE && o != OP_CLAMP01) return false;
+      if (o != OP_MAT3 && o != OP_CBRT && o != OP_CUBE && o != OP_CLAMP01 && o != OP_SRLAB && o != OP_SRLAB_INV)
+        return false;
     }
     return true;
+  }
+  // SrLab2 programs round to FP32 before they round to half floats, as the
+  // interpreter does, so that an image gives the same bits with and without row
+  // padding (left visible, the last matrix's sums round to half floats at once).
+  static constexpr bool srlab() {
+    for (int k = 0; k < n; ++k)
+      if (el_op(el[k]) == OP_SRLAB || el_op(el[k]) == OP_SRLAB_INV) return true;
+    return false;
   }
   // Elements i .. i + 4 composite a loaded layer over the value with straight
   // alpha in and out: premul, load (push), premul, over, unpremul.
@@ -242,6 +251,13 @@ __device__ __forceinline__ void exec(const Uni<P>& u, uint64_t x0, int n, const 
 #pragma unroll
       for (int i = 0; i < kPix; ++i)
         X[i] = make_float4(X[i].x * X[i].x * X[i].x, X[i].y * X[i].y * X[i].y, X[i].z * X[i].z * X[i].z, X[i].w);
+    } else if constexpr (op == OP_SRLAB) {
+#pragma unroll
+      for (int i = 0; i < kPix; ++i) X[i] = make_float4(srlab_nl(X[i].x), srlab_nl(X[i].y), srlab_nl(X[i].z), X[i].w);
+    } else if constexpr (op == OP_SRLAB_INV) {
+#pragma unroll
+      for (int i = 0; i < kPix; ++i)
+        X[i] = make_float4(srlab_nl_inv(X[i].x), srlab_nl_inv(X[i].y), srlab_nl_inv(X[i].z), X[i].w);
     } else if constexpr (op == OP_CLAMP01) {
 #pragma unroll
       for (int i = 0; i < kPix; ++i) X[i] = make_float4(clamp01(X[i].x), clamp01(X[i].y), clamp01(X[i].z), X[i].w);
@@ -265,6 +281,10 @@ __device__ __forceinline__ void exec(const Uni<P>& u, uint64_t x0, int n, const 
       }
     } else if constexpr (op == OP_STORE) {
       constexpr uint32_t F = el_fmt(e);
+      if constexpr (F == FMT_F16 && P::srlab()) {
+#pragma unroll
+        for (int i = 0; i < kPix; ++i) asm volatile("" : "+v"(X[i].x), "+v"(X[i].y), "+v"(X[i].z));
+      }
       if constexpr (P::alpha_byte_passes()) {
         // Alpha bytes straight from the loaded texels (raw[0]: the 4 words).
         encode<F, FULL>((gbyte*)u.base[I] + x0 * fmt_bpp(F), n, X, L, pstride, raw);

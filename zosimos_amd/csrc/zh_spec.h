@@ -27,6 +27,8 @@ constexpr uint16_t sg(uint32_t op, uint32_t fmt = 0, uint32_t push = 0) {
 #define ZH_CBP sg(OP_CBRT, 1)  // cube root of a value the planner proved non-negative
 #define ZH_CU sg(OP_CUBE)
 #define ZH_CL sg(OP_CLAMP01)
+#define ZH_SL sg(OP_SRLAB)
+#define ZH_SI sg(OP_SRLAB_INV)
 #define ZH_PM sg(OP_PREMUL)
 #define ZH_UP sg(OP_UNPREMUL)
 #define ZH_OV sg(OP_OVER)
@@ -52,6 +54,10 @@ constexpr uint16_t sg(uint32_t op, uint32_t fmt = 0, uint32_t push = 0) {
   X(oklab_enc_s8h, ZH_LD(ZH_S8), ZH_M, ZH_CB, ZH_M, ZH_ST(ZH_H))                                          \
   X(oklab_enc_s8hp, ZH_LD(ZH_S8), ZH_M, ZH_CBP, ZH_M, ZH_ST(ZH_H))                                        \
   X(oklab_dec_hs8, ZH_LD(ZH_H), ZH_M, ZH_CU, ZH_M, ZH_CL, ZH_ST(ZH_S8))                                   \
+  /* SrLab2: round trip, to, from */                                                                      \
+  X(srlab_rt_s8, ZH_LD(ZH_S8), ZH_M, ZH_SL, ZH_M, ZH_SI, ZH_M, ZH_CL, ZH_ST(ZH_S8))                       \
+  X(srlab_enc_s8h, ZH_LD(ZH_S8), ZH_M, ZH_SL, ZH_M, ZH_ST(ZH_H))                                          \
+  X(srlab_dec_hs8, ZH_LD(ZH_H), ZH_M, ZH_SI, ZH_M, ZH_CL, ZH_ST(ZH_S8))                                   \
   /* colour matrices */                                                                                  \
   X(mat_s8s8, ZH_LD(ZH_S8), ZH_M, ZH_ST(ZH_S8))                                                           \
   X(mat_hh, ZH_LD(ZH_H), ZH_M, ZH_ST(ZH_H))                                                               \
