@@ -1055,7 +1055,7 @@ class Pool:
         """A copy of the host bytes (``PoolImage::as_bytes``, pool.rs:669)."""
         p, n = ctypes.c_void_p(), ctypes.c_uint64()
         _check(self._lib.zh_pool_host_bytes(self._h, key, ctypes.byref(p), ctypes.byref(n)))
-        return np.frombuffer(ctypes.string_at(p.value, n.value), dtype=np.uint8).copy()
+        return np.frombuffer((ctypes.c_uint8 * n.value).from_address(p.value), dtype=np.uint8).copy()
 
     def device_ptr(self, key: int) -> int:
         img = ctypes.c_void_p()

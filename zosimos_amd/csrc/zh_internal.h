@@ -156,7 +156,7 @@ struct zh_context {
   bool own_stream = false;
   void* d_lut = nullptr;         // zh::Luts (8-bit sRGB tables)
   int cus = 256;                 // compute units of the device
-  uint32_t* d_error = nullptr;   // kernel error flag
+  uint32_t* d_error = nullptr;   // kernel error flag (mapped host memory)
   void* scratch = nullptr;       // the device's static scratch (zh_program_launch_static)
   size_t scratch_bytes = 0;
   // Images and programs hold the context; zh_context_destroy of a context

@@ -44,7 +44,19 @@ struct DeviceBuf {
   DeviceBuf& operator=(const DeviceBuf&) = delete;
 };
 typedef std::shared_ptr<DeviceBuf> DevPtr;
-typedef std::shared_ptr<std::vector<uint8_t>> HostPtr;
+// Host bytes of an image, not cleared first: every holder writes all of them
+// before it publishes them.
+class HostBytes {
+ public:
+  explicit HostBytes(size_t n) : p_(new uint8_t[n]), n_(n) {}
+  uint8_t* data() { return p_.get(); }
+  size_t size() const { return n_; }
+
+ private:
+  std::unique_ptr<uint8_t[]> p_;
+  size_t n_;
+};
+typedef std::shared_ptr<HostBytes> HostPtr;
 
 struct PoolImage {
   zh_descriptor desc{};
@@ -150,7 +162,7 @@ zh_status zh_pool_insert_host(zh_pool* pool, const zh_descriptor* desc, const vo
   if (row_stride == 0) row_stride = row;
   if (row_stride < row) return fail(ZH_ERR_INVALID_ARGUMENT, "row stride shorter than a row");
   im.kind = ZH_IMAGE_HOST;
-  im.host = std::make_shared<std::vector<uint8_t>>(row * im.desc.height);
+  im.host = std::make_shared<HostBytes>(row * im.desc.height);
   for (uint32_t y = 0; y < im.desc.height; ++y)
     std::memcpy(im.host->data() + row * y, static_cast<const uint8_t*>(bytes) + row_stride * y, row);
   *key = pool->next++;
@@ -243,7 +255,7 @@ zh_status zh_pool_download(zh_pool* pool, zh_pool_key key) {
   PoolImage& im = it->second;
   if (im.kind == ZH_IMAGE_HOST) return ZH_OK;
   if (im.kind != ZH_IMAGE_HIP_BUFFER) return fail(ZH_ERR_INVALID_ARGUMENT, "pool image has no data to download");
-  HostPtr host = std::make_shared<std::vector<uint8_t>>(tight_stride(im.desc) * im.desc.height);
+  HostPtr host = std::make_shared<HostBytes>(tight_stride(im.desc) * im.desc.height);
   zh_status st = zh_image_download(im.dev->img, host->data(), 0);
   if (st == ZH_OK) st = zh_sync(im.dev->img->ctx);
   if (st != ZH_OK) return st;
@@ -497,7 +509,7 @@ zh_status zh_execution_retire_output(zh_execution* e, uint32_t slot, int32_t to_
     im.desc = sl.dev->img->desc;
     sl.dev.reset();
   } else {
-    HostPtr host = std::make_shared<std::vector<uint8_t>>(tight_stride(im.desc) * im.desc.height);
+    HostPtr host = std::make_shared<HostBytes>(tight_stride(im.desc) * im.desc.height);
     zh_status st = zh_image_download(sl.dev->img, host->data(), 0);
     if (st == ZH_OK) st = zh_sync(ctx);
     if (st != ZH_OK) return st;

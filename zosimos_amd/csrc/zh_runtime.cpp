@@ -136,10 +136,11 @@ zh_status zh_context_create(int32_t device, void* stream, zh_context** out) {
   srgb_tables(&lut);
   e = hipMalloc(&ctx->d_lut, sizeof(lut));
   if (e == hipSuccess) e = hipDeviceGetAttribute(&ctx->cus, hipDeviceAttributeMultiprocessorCount, device);
-  if (e == hipSuccess) e = hipMalloc(&ctx->d_error, sizeof(uint32_t));
+  // Mapped host memory: zh_sync reads the flag without a copy of its own (12
+  // us); a kernel writes it only where it fails.
+  if (e == hipSuccess) e = hipHostMalloc(&ctx->d_error, sizeof(uint32_t), hipHostMallocDefault);
   if (e == hipSuccess) e = hipMemcpy(ctx->d_lut, &lut, sizeof(lut), hipMemcpyHostToDevice);
-  uint32_t zero = 0;
-  if (e == hipSuccess) e = hipMemcpy(ctx->d_error, &zero, sizeof(zero), hipMemcpyHostToDevice);
+  if (e == hipSuccess) *ctx->d_error = 0;
   if (e == hipSuccess) e = zh_set_resample_lds(kTileLdsBytes);
   // The device address of the static scratch, resolved once per device
   // with the device current (zh_program_launch_static).
@@ -156,7 +157,7 @@ static void context_teardown(zh_context* ctx) {
   hipSetDevice(ctx->device);
   if (ctx->stream) hipStreamSynchronize(ctx->stream);
   if (ctx->d_lut) hipFree(ctx->d_lut);
-  if (ctx->d_error) hipFree(ctx->d_error);
+  if (ctx->d_error) hipHostFree(ctx->d_error);
   if (ctx->own_stream) hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -183,11 +184,9 @@ zh_status zh_sync(zh_context* ctx) {
   if (!ctx) return fail(ZH_ERR_INVALID_ARGUMENT, "null context");
   ZH_HIP(hipSetDevice(ctx->device));
   ZH_HIP(hipStreamSynchronize(ctx->stream));
-  uint32_t flag = 0;
-  ZH_HIP(hipMemcpy(&flag, ctx->d_error, sizeof(flag), hipMemcpyDeviceToHost));
-  if (flag) {
-    uint32_t zero = 0;
-    hipMemcpy(ctx->d_error, &zero, sizeof(zero), hipMemcpyHostToDevice);
+  volatile uint32_t* flag = ctx->d_error;
+  if (*flag) {
+    *flag = 0;
     return fail(ZH_ERR_UNSUPPORTED, "a kernel met a tile larger than its planned LDS box");
   }
   return ZH_OK;
