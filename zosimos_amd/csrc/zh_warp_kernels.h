@@ -378,7 +378,7 @@ __device__ __forceinline__ void tap_weights_inside(const LayerArgs& a, const Lan
   }
 }
 
-template <class V, bool SEP>
+template <class V, bool SEP, bool INSIDE>
 __device__ __forceinline__ void layer_taps(const LayerArgs& a, const LaneMap& mp, bool inside, int n, Px& X,
                                            const Luts* L) {
   typedef typename RawT<V::F>::type R;
@@ -387,7 +387,7 @@ __device__ __forceinline__ void layer_taps(const LayerArgs& a, const LaneMap& mp
   typedef typename PairT<B <= 8 ? B : 8>::type PR;
   uint32_t off[kPix][4];
   float w[kPix][4];
-  if (inside)  // uniform
+  if (INSIDE && inside)  // uniform
     tap_weights_inside<V, SEP>(a, mp, off, w);
   else if (!tap_weights<V, SEP>(a, mp, n, off, w))
     return;
@@ -434,7 +434,7 @@ __device__ __forceinline__ void layer_taps(const LayerArgs& a, const LaneMap& mp
 // lane (lx, ly) owns pixels x = tx * tile_w + lx + k * lanes_x (k < kPix) of
 // row ty * tile_h + ly, so every load and store instruction covers runs of
 // lanes_x adjacent pixels.
-template <class V>
+template <class V, bool INSIDE = true>
 __device__ __forceinline__ void warp_tile(CDesc d, uint32_t tx, uint32_t ty, const Luts* L) {
   typedef typename V::Post Post;
   typedef typename RawT<V::F>::type R;
@@ -474,7 +474,7 @@ __device__ __forceinline__ void warp_tile(CDesc d, uint32_t tx, uint32_t ty, con
     // SEP variant only when every layer has one) are separable: the lane's
     // pixels share one source row pair, computed once.
     const LaneMap mp = lane_map<V::SEP>(Ly, tx * (uint32_t)TW, ty * (uint32_t)TH, lx, ly, lanes_x);
-    layer_taps<V, V::SEP>(a, mp, ((lmask >> (8 + l)) & 1u) != 0, n, X, L);
+    layer_taps<V, V::SEP, INSIDE>(a, mp, ((lmask >> (8 + l)) & 1u) != 0, n, X, L);
   }
 
   if (n == 0) return;
@@ -861,7 +861,7 @@ __device__ __forceinline__ Deal deal_tiles(uint32_t total, uint32_t run) {
   return Deal{v * run, 1u, min(v * run + run, total)};
 }
 
-template <class V>
+template <class V, bool INSIDE = true>
 __device__ __forceinline__ void warp_stage(const StageDesc* dd, uint32_t run) {
   const CDesc d = as_const(dd);
   __shared__ Luts luts;
@@ -873,7 +873,7 @@ __device__ __forceinline__ void warp_stage(const StageDesc* dd, uint32_t run) {
   for (uint32_t t = q.first; t < q.end; t += q.step) {
     uint32_t tx, ty;
     tile_xy(d, t, tx, ty);
-    warp_tile<V>(d, tx, ty, &luts);
+    warp_tile<V, INSIDE>(d, tx, ty, &luts);
   }
 }
 
