@@ -473,7 +473,7 @@ typedef void (*BoxKernel)(const StageDesc*, uint32_t);
 #define ZH_COMMA ,
 
 static BoxKernel box_kernel(uint32_t src, uint32_t dst, bool pow) {
-  // Sources whose transfer is a power function per pixel go through SRC_ANY.
+  // Wide sources whose transfer is a power function per pixel take POW.
   if (src == SRC_TABLE) { ZH_BY_DST(k_box3, dst, pow, SRC_TABLE ZH_COMMA) }
   if (src == SRC_F16) { ZH_BY_DST(k_box3, dst, pow, SRC_F16 ZH_COMMA) }
   if (src == SRC_F32) { ZH_BY_DST(k_box3, dst, pow, SRC_F32 ZH_COMMA) }

@@ -252,6 +252,7 @@ struct zh_program {
   // nothing is freed.
   uint8_t* arena = nullptr;
   size_t arena_size = 0, arena_used = 0;
+  bool no_masks = false;  // warp stages test their layers per tile
   std::vector<zh::StageDesc> h_stage_vec;
   // User stages: the loaded kernel and the device copy of the shader data,
   // per entry of plan.dynamics.

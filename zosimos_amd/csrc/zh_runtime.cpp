@@ -483,10 +483,10 @@ static uint32_t tile_meets_layer(const Layer& L, double ex0, double ey0, double 
 }
 
 // The tile-layer masks of warp stage s for its current tile shape (host
-// computation, uploaded once; the kernels then read one byte per tile).
+// computation, uploaded once; the kernels then read two bytes per tile).
 static zh_status tile_layer_masks(zh_program* p, size_t s) {
   StageDesc& d = p->plan.stages[s].desc;
-  if (d.kind != STAGE_RESAMPLE || d.variant < 0 || d.n_layers == 0 || d.n_layers > 8) return ZH_OK;
+  if (d.kind != STAGE_RESAMPLE || d.variant < 0 || d.n_layers == 0 || d.n_layers > 8 || p->no_masks) return ZH_OK;
   if (p->d_tile_layers.size() < p->plan.stages.size()) {
     p->d_tile_layers.resize(p->plan.stages.size(), nullptr);
     p->tile_layer_words.resize(p->plan.stages.size(), 0);
@@ -1456,24 +1456,32 @@ zh_status zh_program_launch_static(zh_context* ctx, const zh_descriptor* texture
   if (!ctx->scratch || ctx->scratch_bytes == 0)
     return fail(ZH_ERR_HIP, "the device's static scratch was not resolved at context creation");
   ZH_HIP(hipSetDevice(ctx->device));
-  zh_program prog;
-  zh_program* p = &prog;
-  // No hipGraph: instantiating one allocates.
-  zh_status st = init_program(p, ctx, textures, num_textures, ops, num_ops, flags | ZH_PLAN_NO_GRAPH);
-  if (st != ZH_OK) return st;
-  // Loading a user kernel's code object allocates.
-  if (!p->plan.dynamics.empty())
-    return fail(ZH_ERR_UNSUPPORTED, "user stage kernels cannot run from the static scratch (loading them allocates)");
   // An earlier call's kernels on this stream may still read the scratch:
   // let them finish before its tables are overwritten.
   ZH_HIP(hipStreamSynchronize(ctx->stream));
-  p->arena = static_cast<uint8_t*>(ctx->scratch);
-  p->arena_size = ctx->scratch_bytes;
-  p->arena_used = 0;
-  st = alloc_device(p);
-  if (st == ZH_OK) st = bind(p, bindings, num_bindings);
-  if (st == ZH_OK) st = launch_all(p);
-  free_device(p);  // host side only: the tables stay in the scratch for the queued kernels
+  // Programs whose tables overflow the scratch try once more without the
+  // warp stages' tile masks, which the kernels can do without.
+  zh_status st = ZH_OK;
+  for (bool masks : {true, false}) {
+    zh_program prog;
+    zh_program* p = &prog;
+    // No hipGraph: instantiating one allocates.
+    st = init_program(p, ctx, textures, num_textures, ops, num_ops, flags | ZH_PLAN_NO_GRAPH);
+    if (st != ZH_OK) return st;
+    // Loading a user kernel's code object allocates.
+    if (!p->plan.dynamics.empty())
+      return fail(ZH_ERR_UNSUPPORTED, "user stage kernels cannot run from the static scratch (loading them allocates)");
+    p->arena = static_cast<uint8_t*>(ctx->scratch);
+    p->arena_size = ctx->scratch_bytes;
+    p->arena_used = 0;
+    p->no_masks = !masks;
+    st = alloc_device(p);
+    const bool again = st == ZH_ERR_OUT_OF_MEMORY && masks;
+    if (st == ZH_OK) st = bind(p, bindings, num_bindings);
+    if (st == ZH_OK) st = launch_all(p);
+    free_device(p);  // host side only: the tables stay in the scratch for the queued kernels
+    if (!again) break;
+  }
   return st;
 }
 

@@ -225,9 +225,11 @@ struct StageDesc {
   // meets the tile and a byte of those whose source holds every tap of it, two
   // tiles per word (bit l: layer l); null: the kernel tests each layer itself.
   const uint32_t* tile_layers;
-  TableDesc table[2];         // any-format kernels: the decode tables of their loads
   uint32_t* error_flag;       // set to 1 by a kernel that met an impossible case
-  Layer layer[kMaxLayers];
+  union {
+    Layer layer[kMaxLayers];  // resample
+    TableDesc table[2];       // pointwise, any-format kernels: the decode tables of their loads
+  };
   Slot slot[kMaxSlots];
   Instr code[kMaxInstr];
   float params[kMaxParams];
