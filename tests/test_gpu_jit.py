@@ -132,3 +132,35 @@ def test_unregistered_warp_form_runs_a_compiled_kernel(ctx):
         diff = np.abs(out[o].astype(int) - interp[o].astype(int))
         report(f"jitw_vs_interpreter_{w}x{h}", max_code_diff=int(diff.max()), equal=float((diff == 0).mean()))
         assert diff.max() <= 1
+
+
+@pytest.mark.parametrize("degrees", [0.0, 25.0])
+def test_two_half_float_sources_hold_their_registers(ctx, degrees):
+    """'over' of two RGBA16F images under an affine map, alone and as a batch:
+    the compiled kernels (separable and general maps) spill no register, and
+    each result is within one f16 ulp of the FP64 oracle (1e-6 absolute near
+    zero)."""
+    from oracle import color as C
+    rng = np.random.default_rng(21)
+    for sizes in ([(130, 70)], [(130, 70), (64, 33)]):
+        cmd, inputs, host, outputs, want = z.CommandBuffer(), {}, {}, {}, {}
+        for w, h in sizes:
+            d = z.Descriptor.rgba16f_linear(w, h)
+            a, b = cmd.input(d), cmd.input(d)
+            ab = cmd.blend(a, z.Rectangle(0, 0, w, h), b)
+            aff = W.about_centre(w, h, 0.8, np.deg2rad(degrees))
+            o, od = cmd.output(cmd.affine(cmd.solid_rgba(d, (0, 0, 0, 0)), aff, ab))
+            for r in (a, b):
+                inputs[r], host[r] = d, W.random_rgba16f(rng, w, h)
+            outputs[o] = od
+            A, B = (C.premultiply(PL.f16_image(host[r], w, h)) for r in (a, b))
+            want[o] = C.unpremultiply(C.bilinear_affine(C.over(B, A), PL.mat_f32(aff.transformation), (h, w)))
+        out, exe = run(ctx, cmd, inputs, host, outputs)
+        text = exe.describe()
+        assert "\njitw#" in text and "unavailable" not in text, text
+        assert "scratch" not in text, text
+        for o, v in want.items():
+            got = np.asarray(out[o]).reshape(-1).view(np.float16).reshape(v.shape)
+            ulp = np.abs(got.view(np.int16).astype(int) - C.encode_f16(v).view(np.int16).astype(int))
+            ulp = np.where(np.abs(got.astype(np.float64) - v) <= 1e-6, 0, ulp)
+            assert np.where(v[..., 3:] > 1e-3, ulp, 0).max() <= 1

@@ -107,18 +107,18 @@ std::string source_for(const JitEntry& e) {
            "typedef zh::spec::Prog<" + list + "> P;\n" +
            k + "zh_jit_stage(const zh::StageDesc* d) { zh::spec::spec_stage<P>(d); }\n" +
            k + "zh_jit_batch(const zh::BatchDesc* b) { zh::spec::spec_batch<P>(b); }\n";
-  // As zh_warp.hip: half-float sources are bounded to the registers of 5 waves.
-  const std::string kw = std::string("extern \"C\" __global__ __launch_bounds__(256, ") +
-                         (e.fmt == FMT_F16 ? "5" : "1") + ") void ";
   const std::string form = std::to_string(e.src) + "u, " + std::to_string(e.fmt) + "u, " + (e.mat ? "true" : "false") +
                            ", zh::spec::Prog<" + list + ">, ";
+  auto kw = [](const char* v) {
+    return std::string("extern \"C\" __global__ __launch_bounds__(256, zh::spec::min_waves<") + v + ">()) void ";
+  };
   std::string src = "#include \"zh_warp_kernels.h\"\n"
                     "typedef zh::spec::Warp<" + form + "false> V;\n"
                     "typedef zh::spec::Warp<" + form + "true> VS;\n" +
-                    kw + "zh_jit_warp(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<V>(d, r); }\n" +
-                    kw + "zh_jit_warp_sep(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<VS>(d, r); }\n" +
-                    kw + "zh_jit_warp_batch(const zh::BatchDesc* b, uint32_t r) { zh::spec::warp_batch<V>(b, r); }\n" +
-                    kw + "zh_jit_warp_batch_sep(const zh::BatchDesc* b, uint32_t r) { zh::spec::warp_batch<VS>(b, r); }\n";
+                    kw("V") + "zh_jit_warp(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<V>(d, r); }\n" +
+                    kw("VS") + "zh_jit_warp_sep(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<VS>(d, r); }\n" +
+                    kw("V") + "zh_jit_warp_batch(const zh::BatchDesc* b, uint32_t r) { zh::spec::warp_batch<V>(b, r); }\n" +
+                    kw("VS") + "zh_jit_warp_batch_sep(const zh::BatchDesc* b, uint32_t r) { zh::spec::warp_batch<VS>(b, r); }\n";
   if (e.src == WSRC_ONE)
     src += k + "zh_jit_warp_staged(const zh::StageDesc* d, uint32_t) { zh::spec::warp_staged_stage<VS>(d); }\n" +
            k + "zh_jit_warp_batch_staged(const zh::BatchDesc* b, uint32_t) { zh::spec::warp_staged_batch<VS>(b); }\n";

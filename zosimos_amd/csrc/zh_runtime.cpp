@@ -14,6 +14,7 @@
 #include <cstddef>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <set>
 #include <sstream>
@@ -795,6 +796,18 @@ zh_status zh_program_launch_bytes(zh_program* p, uint64_t* bytes, uint32_t max_l
   return ZH_OK;
 }
 
+// ", N bytes of scratch a lane" when one of the kernels spills registers.
+static std::string scratch_of(std::initializer_list<hipFunction_t> fns) {
+  int most = 0;
+  for (hipFunction_t f : fns) {
+    int n = 0;
+    if (!f) continue;
+    if (hipFuncGetAttribute(&n, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, f) == hipSuccess) most = std::max(most, n);
+    else (void)hipGetLastError();
+  }
+  return most ? ", " + std::to_string(most) + " bytes of scratch a lane" : std::string();
+}
+
 zh_status zh_program_describe(zh_program* p, char* buf, size_t len, size_t* needed) {
   if (!p) return fail(ZH_ERR_INVALID_ARGUMENT, "null program");
   std::ostringstream o;
@@ -831,11 +844,19 @@ zh_status zh_program_describe(zh_program* p, char* buf, size_t len, size_t* need
       o << "launch " << i << ": tiles in strips " << p->units[i].strip_w << " tiles wide\n";
   }
   {
-    std::set<int> shown;
+    std::set<int> shown, shown_warp;
     for (size_t i = 0; i < p->plan.stages.size(); ++i) {
       const int j = p->plan.stages[i].jit;
       if (j >= 0 && i < p->jit_stage_fn.size() && p->jit_stage_fn[i] && shown.insert(j).second)
-        o << "jit#" << j << ": compiled at run time in " << jit_compile_seconds(j) << " s\n";
+        o << "jit#" << j << ": compiled at run time in " << jit_compile_seconds(j) << " s"
+          << scratch_of({p->jit_stage_fn[i], p->jit_batch_fn[i]}) << "\n";
+      const StageDesc& d = p->plan.stages[i].desc;
+      if (d.kind != STAGE_RESAMPLE || d.variant < kJitWarpBase || i >= p->jit_stage_fn.size() || !p->jit_stage_fn[i])
+        continue;
+      if (shown_warp.insert(d.variant).second)
+        o << "jitw#" << (d.variant - kJitWarpBase) / 2 << ((d.variant & 1) ? "_sep" : "") << ": compiled at run time in "
+          << jit_compile_seconds((d.variant - kJitWarpBase) / 2) << " s"
+          << scratch_of({p->jit_stage_fn[i], p->jit_batch_fn[i]}) << "\n";
     }
   }
   for (size_t i = 0; i < p->plan.intermediates.size(); ++i) {

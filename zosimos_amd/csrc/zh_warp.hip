@@ -13,12 +13,6 @@
 namespace zh {
 namespace spec {
 
-// Half-float sources: bounded to the registers of 5 waves a SIMD, the scheduler
-// finds an order that holds 6 for most forms (78-80 VGPRs without spills; left
-// free, 84).
-template <class V>
-constexpr int min_waves() { return V::F == FMT_F16 ? 5 : 1; }
-
 template <class V>
 __global__ __launch_bounds__(kBlock, min_waves<V>()) void k_warp(const StageDesc* dd, uint32_t run) {
   warp_stage<V>(dd, run);

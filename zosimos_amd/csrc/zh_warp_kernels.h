@@ -861,6 +861,16 @@ __device__ __forceinline__ Deal deal_tiles(uint32_t total, uint32_t run) {
   return Deal{v * run, 1u, min(v * run + run, total)};
 }
 
+// Waves a SIMD that a form's stage and batch kernels are bounded to, the
+// registered ones and those compiled at run time.  One half-float source:
+// bounded to the registers of 5 waves, the scheduler finds an order that holds 6
+// for the form with a matrix and the separable forms of short post programs
+// (78-80 VGPRs; left free 84, the others 82-88 without spills).  Two of them
+// hold 113 (the raw taps of both): under that bound 17 were spilled (80 bytes of
+// scratch a lane; 3840x2160 rotated 66.3 us, left free 42.0).
+template <class V>
+constexpr int min_waves() { return V::F == FMT_F16 && V::SRC == WSRC_ONE ? 5 : 1; }
+
 template <class V, bool INSIDE = true>
 __device__ __forceinline__ void warp_stage(const StageDesc* dd, uint32_t run) {
   const CDesc d = as_const(dd);
