@@ -164,3 +164,45 @@ def test_two_half_float_sources_hold_their_registers(ctx, degrees):
             ulp = np.abs(got.view(np.int16).astype(int) - C.encode_f16(v).view(np.int16).astype(int))
             ulp = np.where(np.abs(got.astype(np.float64) - v) <= 1e-6, 0, ulp)
             assert np.where(v[..., 3:] > 1e-3, ulp, 0).max() <= 1
+
+
+@pytest.mark.parametrize("degrees", [0.0, 12.0])
+@pytest.mark.parametrize("texel,w,h,few", [
+    ("f16", 63, 15, True), ("f16", 400, 300, True), ("f16", 1024, 256, True), ("f16", 1025, 256, False),
+    ("f32", 63, 15, True), ("f32", 1025, 256, True), ("f32", 1400, 1400, False), ("u8", 400, 300, False)])
+def test_compiled_form_of_few_tiles(ctx, texel, w, h, few, degrees):
+    """Four layers through a compiled form: up to one tile per compute unit
+    (256) of half floats, or a grid resident as a whole of floats, the kernel
+    without a choice of path runs, else the other; within 1 code of the FP64
+    oracle (colour where alpha is above 0.02)."""
+    from oracle import color as C
+    rng = np.random.default_rng([w, h])
+    cmd = z.CommandBuffer()
+    tex, color = {"f16": (W.RGBA16F, W.P3_LINEAR), "f32": (z.Descriptor.rgba32f_linear(1, 1).texel, W.P3_LINEAR),
+                  "u8": (W.RGBA8, W.P3_SRGB)}[texel]
+    d = z.Descriptor(w, h, tex, color)
+    acc = cmd.solid_rgba(d, (0, 0, 0, 0))
+    inputs, host, want = {}, {}, np.zeros((h, w, 4))
+    for k in range(4):
+        a = cmd.input(d)
+        inputs[a] = d
+        if texel == "u8":
+            host[a] = W.random_rgba8(rng, w, h)
+            src = C.decode_u8(PL.u8_image(host[a], w, h), 5)
+        else:
+            host[a] = W.random_rgba16f(rng, w, h)
+            src = PL.f16_image(host[a], w, h)
+            if texel == "f32":
+                host[a] = src.astype(np.float32).view(np.uint8).reshape(-1)
+        aff = W.about_centre(w, h, 0.6 + 0.3 * k, np.deg2rad(degrees * k))
+        acc = cmd.affine(acc, aff, a)
+        want = C.over(C.bilinear_affine(C.premultiply(src), PL.mat_f32(aff.transformation), (h, w)), want)
+    o, od = cmd.output(cmd.color_convert(acc, z.Color.SRGB, W.RGBA8))
+    out, exe = run(ctx, cmd, inputs, host, {o: od})
+    text = exe.describe()
+    assert "[kernel jitw#" in text and ("kernel for few" in text) == few, text
+    assert "scratch" not in text, text
+    straight = C.unpremultiply(want)
+    codes = C.encode_u8(PL.apply3(C.convert_matrix(7, 3, 5), straight), 5)
+    mr, ma, _ = compare_u8(f"jitw_few_{texel}_{w}x{h}_{degrees}", out[o], codes, alpha_ok=straight[..., 3] > 0.02)
+    assert mr <= 1 and ma <= 1

@@ -73,10 +73,10 @@ double jit_compile_seconds(int id);
 // of operations the warp bodies run, and the process-wide id of a form.
 bool jit_warp_supported(const uint16_t* post, int n);
 int jit_warp_form(uint32_t src, uint32_t fmt, uint32_t mat, const uint16_t* post, int n);
-// The general, separable or LDS-staged (separable, one source) stage kernel
-// and batch kernel of form `id`.
-zh_status jit_warp_kernels(int id, bool sep, bool staged, int device, hipFunction_t* stage, hipFunction_t* batch,
-                           std::string* why);
+// The general, separable or LDS-staged (separable, one source) stage kernel,
+// its form for few tiles (null for staged kernels) and batch kernel of form `id`.
+zh_status jit_warp_kernels(int id, bool sep, bool staged, int device, hipFunction_t* stage, hipFunction_t* few,
+                           hipFunction_t* batch, std::string* why);
 // Does form `id` have LDS-staged kernels (one-source forms)?
 bool jit_warp_has_staged(int id);
 // An affine layer-stack form as the warp bodies take it.
@@ -258,9 +258,11 @@ struct zh_program {
   // per entry of plan.dynamics.
   std::vector<hipFunction_t> dyn_fn;
   std::vector<void*> dyn_data;
-  // Run-time kernels per stage (StagePlan::jit): stage and batch forms and
-  // their resident workgroups per CU.
-  std::vector<hipFunction_t> jit_stage_fn, jit_batch_fn;
+  // Run-time kernels per stage (StagePlan::jit): stage form, that for few tiles
+  // (or null), batch form, and their resident workgroups per CU.
+  std::vector<hipFunction_t> jit_stage_fn, jit_few_fn, jit_batch_fn;
+  // Warp stages: tiles up to which the kernel for few runs (zh_warp_few_tiles).
+  std::vector<uint32_t> few_tiles;
   std::vector<uint32_t> jit_resident, jit_batch_resident;
   // The stepped execution (zh_program_start_pool) still launching this
   // program's kernels; other launches wait for it to finish.

@@ -44,6 +44,7 @@ namespace {
 struct JitEntry {
   bool warp = false;
   bool pair = false;  // two warp forms in one grid: the first in src..sig, the second in src2..sig2
+  bool staged = false;  // the LDS-staged kernels of a one-source form
   uint32_t src = 0, fmt = 0, mat = 0;
   std::vector<uint16_t> sig;
   bool sep = false, sep2 = false;
@@ -52,8 +53,9 @@ struct JitEntry {
   bool compiled = false;
   std::string error;  // why the compile failed (compiled and no kernels)
   // Kernels held for the process: pointwise {stage, batch}; warp {stage,
-  // stage of separable maps, batch, batch of separable maps} and, for
-  // one-source forms, the LDS-staged {stage, batch} of separable maps.
+  // stage of separable maps, batch, batch of separable maps} and, for forms
+  // that have one, the kernel for few tiles {general, separable maps}; LDS-staged
+  // {stage, batch} (separable maps).
   std::vector<zh_shader*> kernels;
   double compile_s = 0.0;
 };
@@ -74,12 +76,12 @@ std::string package_dir() {
 }
 
 const char* const kSpecKernels[] = {"zh_jit_stage", "zh_jit_batch"};
-const char* const kWarpKernels[] = {"zh_jit_warp",       "zh_jit_warp_sep",    "zh_jit_warp_batch",
-                                    "zh_jit_warp_batch_sep", "zh_jit_warp_staged", "zh_jit_warp_batch_staged"};
-
+const char* const kWarpKernels[] = {"zh_jit_warp",           "zh_jit_warp_sep", "zh_jit_warp_batch",
+                                    "zh_jit_warp_batch_sep", "zh_jit_warp_few", "zh_jit_warp_few_sep"};
+const char* const kStagedKernels[] = {"zh_jit_warp_staged", "zh_jit_warp_batch_staged"};
 const char* const kPairKernels[] = {"zh_jit_warp_pair"};
 
-int kernel_count(const JitEntry& e) { return e.pair ? 1 : !e.warp ? 2 : e.src == WSRC_ONE ? 6 : 4; }
+int kernel_count(const JitEntry& e) { return e.pair ? 1 : !e.warp || e.staged ? 2 : warp_has_few(e.src, e.fmt) ? 6 : 4; }
 
 std::string prog_list(const std::vector<uint16_t>& sig) {
   std::string list;
@@ -112,16 +114,21 @@ std::string source_for(const JitEntry& e) {
   auto kw = [](const char* v) {
     return std::string("extern \"C\" __global__ __launch_bounds__(256, zh::spec::min_waves<") + v + ">()) void ";
   };
-  std::string src = "#include \"zh_warp_kernels.h\"\n"
-                    "typedef zh::spec::Warp<" + form + "false> V;\n"
-                    "typedef zh::spec::Warp<" + form + "true> VS;\n" +
-                    kw("V") + "zh_jit_warp(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<V>(d, r); }\n" +
-                    kw("VS") + "zh_jit_warp_sep(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<VS>(d, r); }\n" +
-                    kw("V") + "zh_jit_warp_batch(const zh::BatchDesc* b, uint32_t r) { zh::spec::warp_batch<V>(b, r); }\n" +
-                    kw("VS") + "zh_jit_warp_batch_sep(const zh::BatchDesc* b, uint32_t r) { zh::spec::warp_batch<VS>(b, r); }\n";
-  if (e.src == WSRC_ONE)
-    src += k + "zh_jit_warp_staged(const zh::StageDesc* d, uint32_t) { zh::spec::warp_staged_stage<VS>(d); }\n" +
+  const std::string types = "#include \"zh_warp_kernels.h\"\n"
+                            "typedef zh::spec::Warp<" + form + "false> V;\n"
+                            "typedef zh::spec::Warp<" + form + "true> VS;\n";
+  if (e.staged)
+    return types +
+           k + "zh_jit_warp_staged(const zh::StageDesc* d, uint32_t) { zh::spec::warp_staged_stage<VS>(d); }\n" +
            k + "zh_jit_warp_batch_staged(const zh::BatchDesc* b, uint32_t) { zh::spec::warp_staged_batch<VS>(b); }\n";
+  std::string src =
+      types + kw("V") + "zh_jit_warp(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<V>(d, r); }\n" +
+      kw("VS") + "zh_jit_warp_sep(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<VS>(d, r); }\n" +
+      kw("V") + "zh_jit_warp_batch(const zh::BatchDesc* b, uint32_t r) { zh::spec::warp_batch<V>(b, r); }\n" +
+      kw("VS") + "zh_jit_warp_batch_sep(const zh::BatchDesc* b, uint32_t r) { zh::spec::warp_batch<VS>(b, r); }\n";
+  if (warp_has_few(e.src, e.fmt))
+    src += k + "zh_jit_warp_few(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<V, false>(d, r); }\n" +
+           k + "zh_jit_warp_few_sep(const zh::StageDesc* d, uint32_t r) { zh::spec::warp_stage<VS, false>(d, r); }\n";
   return src;
 }
 
@@ -157,7 +164,7 @@ void compile(JitEntry& e) {
   std::vector<char> code(n);
   hiprtcGetCode(prog, code.data());
   hiprtcDestroyProgram(&prog);
-  const char* const* names = e.pair ? kPairKernels : e.warp ? kWarpKernels : kSpecKernels;
+  const char* const* names = e.pair ? kPairKernels : e.staged ? kStagedKernels : e.warp ? kWarpKernels : kSpecKernels;
   const int count = kernel_count(e);
   for (int i = 0; i < count; ++i) {
     zh_shader* k = nullptr;
@@ -175,7 +182,7 @@ int find_or_add(const JitEntry& want) {
   std::vector<JitEntry>& es = entries();
   for (size_t i = 0; i < es.size(); ++i) {
     const JitEntry& e = es[i];
-    if (e.warp == want.warp && e.pair == want.pair && e.src == want.src && e.fmt == want.fmt && e.mat == want.mat &&
+    if (e.warp == want.warp && e.pair == want.pair && e.staged == want.staged && e.src == want.src && e.fmt == want.fmt && e.mat == want.mat &&
         e.sig == want.sig && e.sep == want.sep && e.src2 == want.src2 && e.fmt2 == want.fmt2 &&
         e.mat2 == want.mat2 && e.sig2 == want.sig2 && e.sep2 == want.sep2)
       return (int)i;
@@ -264,15 +271,43 @@ int jit_warp_form(uint32_t src, uint32_t fmt, uint32_t mat, const uint16_t* post
   return find_or_add(e);
 }
 
-zh_status jit_warp_kernels(int id, bool sep, bool staged, int device, hipFunction_t* stage, hipFunction_t* batch,
-                           std::string* why) {
-  hipFunction_t f[2] = {nullptr, nullptr};
-  if (staged && !jit_warp_has_staged(id)) return fail(ZH_ERR_INVALID_ARGUMENT, "run-time warp form without staged tiles");
-  zh_status st = staged ? kernels_of(id, true, {4, 5}, device, f, why)
-                 : sep  ? kernels_of(id, true, {1, 3}, device, f, why)
-                        : kernels_of(id, true, {0, 2}, device, f, why);
+zh_status jit_warp_kernels(int id, bool sep, bool staged, int device, hipFunction_t* stage, hipFunction_t* few,
+                           hipFunction_t* batch, std::string* why) {
+  *few = nullptr;
+  hipFunction_t f[3] = {nullptr, nullptr, nullptr};
+  zh_status st;
+  if (staged) {
+    if (!jit_warp_has_staged(id)) return fail(ZH_ERR_INVALID_ARGUMENT, "run-time warp form without staged tiles");
+    int twin;
+    {
+      std::lock_guard<std::mutex> lock(g_mu);
+      const JitEntry& e = entries()[(size_t)id];
+      JitEntry t;
+      t.warp = true;
+      t.staged = true;
+      t.src = e.src;
+      t.fmt = e.fmt;
+      t.mat = e.mat;
+      t.sig = e.sig;
+      twin = find_or_add(t);
+    }
+    st = kernels_of(twin, true, {0, 1}, device, f, why);
+    *stage = f[0];
+    *batch = f[1];
+    return st;
+  }
+  bool few_too;
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    const std::vector<JitEntry>& es = entries();
+    few_too = id >= 0 && id < (int)es.size() && warp_has_few(es[(size_t)id].src, es[(size_t)id].fmt);
+  }
+  st = sep ? kernels_of(id, true, {1, 3}, device, f, why) : kernels_of(id, true, {0, 2}, device, f, why);
+  if (st == ZH_OK && few_too)
+    st = sep ? kernels_of(id, true, {5}, device, f + 2, why) : kernels_of(id, true, {4}, device, f + 2, why);
   *stage = f[0];
   *batch = f[1];
+  *few = f[2];
   return st;
 }
 

@@ -20,6 +20,7 @@
 #include <sstream>
 
 #include "zh_internal.h"
+#include "zh_spec.h"
 
 extern "C" {
 hipError_t zh_launch_pointwise(const zh::StageDesc* d_dev, uint32_t width, uint32_t height, int flat, int fast,
@@ -34,7 +35,7 @@ hipError_t zh_launch_spec(int index, const zh::StageDesc* d_dev, uint32_t width,
 hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, hipStream_t stream);
 void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int staged, uint32_t* blocks,
                   uint32_t* run);
-hipError_t zh_launch_warp(int index, int staged, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
+hipError_t zh_launch_warp(int index, int staged, int few, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
                           uint32_t per_cu, hipStream_t stream);
 hipError_t zh_launch_warp_batch(int index, int staged, const zh::BatchDesc* b_dev, uint32_t total_tiles,
                                 uint32_t cus, uint32_t per_cu, hipStream_t stream);
@@ -613,6 +614,8 @@ static zh_status alloc_device(zh_program* p) {
   // static scratch: loading a code object allocates).  A kernel that cannot
   // be had leaves its stage on the interpreter, and the description says why.
   p->jit_stage_fn.assign(p->plan.stages.size(), nullptr);
+  p->jit_few_fn.assign(p->plan.stages.size(), nullptr);
+  p->few_tiles.assign(p->plan.stages.size(), 0);
   p->jit_batch_fn.assign(p->plan.stages.size(), nullptr);
   p->jit_resident.assign(p->plan.stages.size(), 1);
   p->jit_batch_resident.assign(p->plan.stages.size(), 1);
@@ -622,10 +625,10 @@ static zh_status alloc_device(zh_program* p) {
       // A run-time warp form; without it the stage runs on the resample
       // interpreter, whose kernels accept the same tiles.
       std::string why;
-      hipFunction_t f = nullptr, fb = nullptr;
+      hipFunction_t f = nullptr, ff = nullptr, fb = nullptr;
       const int id = (sp.desc.variant - kJitWarpBase) / 2;
       const bool sep = (sp.desc.variant & 1) != 0;
-      if (p->arena || jit_warp_kernels(id, sep, sp.staged, ctx->device, &f, &fb, &why) != ZH_OK) {
+      if (p->arena || jit_warp_kernels(id, sep, sp.staged, ctx->device, &f, &ff, &fb, &why) != ZH_OK) {
         sp.desc.variant = -1;
         sp.staged = false;
         const size_t k = sp.text.rfind(" [kernel jitw#");
@@ -641,8 +644,17 @@ static zh_status alloc_device(zh_program* p) {
       if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&n, fb, kBlock, 0) == hipSuccess && n > 0)
         p->jit_batch_resident[s] = (uint32_t)n;
       p->jit_stage_fn[s] = f;
+      p->jit_few_fn[s] = ff;
+      WarpForm form;
+      if (ff && warp_form_of(sp.desc.variant, &form))
+        p->few_tiles[s] = zh_warp_few_tiles(form.src, form.fmt, p->jit_resident[s], (uint32_t)ctx->cus);
       p->jit_batch_fn[s] = fb;
       continue;
+    }
+    if (sp.desc.kind == STAGE_RESAMPLE && sp.desc.variant >= 0 && !sp.staged) {
+      WarpForm form;
+      if (warp_form_of(sp.desc.variant, &form))
+        p->few_tiles[s] = zh_warp_few_tiles(form.src, form.fmt, zh_warp_resident(sp.desc.variant, 0), (uint32_t)ctx->cus);
     }
     if (sp.jit < 0) continue;
     std::string why;
@@ -796,6 +808,12 @@ zh_status zh_program_launch_bytes(zh_program* p, uint64_t* bytes, uint32_t max_l
   return ZH_OK;
 }
 
+// Does warp stage s run its form's kernel for few tiles?
+static bool runs_few(const zh_program* p, size_t s) {
+  const StageDesc& d = p->plan.stages[s].desc;
+  return s < p->few_tiles.size() && d.tiles_x * d.tiles_y <= p->few_tiles[s];
+}
+
 // ", N bytes of scratch a lane" when one of the kernels spills registers.
 static std::string scratch_of(std::initializer_list<hipFunction_t> fns) {
   int most = 0;
@@ -837,7 +855,11 @@ zh_status zh_program_describe(zh_program* p, char* buf, size_t len, size_t* need
                                                  : " as one tile queue\n");
     }
     const StageDesc& d0 = p->plan.stages[u.ids[0]].desc;
-    if (d0.kind == STAGE_RESAMPLE) o << "launch " << i << ": tiles " << d0.tile_w << "x" << d0.tile_h << "\n";
+    if (d0.kind == STAGE_RESAMPLE) {
+      o << "launch " << i << ": tiles " << d0.tile_w << "x" << d0.tile_h;
+      if (!u.batch && d0.variant >= 0 && runs_few(p, u.ids[0])) o << ", kernel for few";
+      o << "\n";
+    }
     if (p->units[i].blocks_per_cu)
       o << "launch " << i << ": " << p->units[i].blocks_per_cu << " workgroups per CU\n";
     if (p->units[i].strip_w)
@@ -856,7 +878,7 @@ zh_status zh_program_describe(zh_program* p, char* buf, size_t len, size_t* need
       if (shown_warp.insert(d.variant).second)
         o << "jitw#" << (d.variant - kJitWarpBase) / 2 << ((d.variant & 1) ? "_sep" : "") << ": compiled at run time in "
           << jit_compile_seconds((d.variant - kJitWarpBase) / 2) << " s"
-          << scratch_of({p->jit_stage_fn[i], p->jit_batch_fn[i]}) << "\n";
+          << scratch_of({p->jit_stage_fn[i], p->jit_few_fn[i], p->jit_batch_fn[i]}) << "\n";
     }
   }
   for (size_t i = 0; i < p->plan.intermediates.size(); ++i) {
@@ -1247,17 +1269,18 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
     }
     case STAGE_RESAMPLE:
       if (first < p->variant.size() && p->variant[first] == 3 && sp.desc.variant >= kJitWarpBase) {
-        // A run-time warp form: the grid of zh_launch_warp.
+        // A run-time warp form: the grid and kernel of zh_launch_warp.
+        const uint32_t tiles = sp.desc.tiles_x * sp.desc.tiles_y, cus = (uint32_t)p->ctx->cus;
         uint32_t blocks, run;
-        zh_warp_grid(sp.desc.tiles_x * sp.desc.tiles_y, p->jit_resident[first], (uint32_t)p->ctx->cus, u.blocks_per_cu,
-                     sp.staged, &blocks, &run);
+        zh_warp_grid(tiles, p->jit_resident[first], cus, u.blocks_per_cu, sp.staged, &blocks, &run);
         if (blocks == 0) break;
+        const hipFunction_t fn = runs_few(p, first) ? p->jit_few_fn[first] : p->jit_stage_fn[first];
         const StageDesc* dp = d;
         void* args[] = {&dp, &run};
-        ZH_HIP(hipModuleLaunchKernel(p->jit_stage_fn[first], blocks, 1, 1, kBlock, 1, 1, 0, s, args, nullptr));
+        ZH_HIP(hipModuleLaunchKernel(fn, blocks, 1, 1, kBlock, 1, 1, 0, s, args, nullptr));
       } else if (first < p->variant.size() && p->variant[first] == 3) {
-        ZH_HIP(zh_launch_warp(sp.desc.variant, sp.staged, d, sp.desc.tiles_x * sp.desc.tiles_y, (uint32_t)p->ctx->cus,
-                              u.blocks_per_cu, s));
+        ZH_HIP(zh_launch_warp(sp.desc.variant, sp.staged, runs_few(p, first), d, sp.desc.tiles_x * sp.desc.tiles_y,
+                              (uint32_t)p->ctx->cus, u.blocks_per_cu, s));
       } else if (first < p->variant.size() && p->variant[first] == 9) {
         ZH_HIP(zh_launch_move(sp.move, d, sp.desc.width, sp.desc.height, s));
       } else {

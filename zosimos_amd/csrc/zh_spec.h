@@ -89,6 +89,13 @@ constexpr uint16_t sg(uint32_t op, uint32_t fmt = 0, uint32_t push = 0) {
 // X(name, source form, F, mat3 in the source program, post elements...)
 enum WarpSrc : uint32_t { WSRC_ONE = 0, WSRC_OVER2 = 1 };
 
+// Has a form a second stage kernel, without the choice of path by the host's
+// masks, for stages of few tiles?  There every instruction's latency shows (one
+// wave a SIMD), and border tests are cheaper than the choice: one source of half
+// floats or of floats.  Of 8-bit texels and of two sources the choice is as fast
+// or faster (four RGBA8 layers 400x300: 9.2 us against 9.4).
+constexpr bool warp_has_few(uint32_t src, uint32_t fmt) { return src == WSRC_ONE && (fmt == FMT_F16 || fmt == FMT_F32); }
+
 #define ZH_WARP_LIST(X)                                                                        \
   X(w_over2_s8, WSRC_OVER2, ZH_S8, 0, ZH_UP, ZH_ST(ZH_S8))                                      \
   X(w_s8m_s8, WSRC_ONE, ZH_S8, 1, ZH_UP, ZH_ST(ZH_S8))                                          \
@@ -110,6 +117,15 @@ const char* zh_spec_name(int index);
 // for axis-aligned maps.
 int zh_warp_lookup(uint32_t src, uint32_t fmt, uint32_t mat, const uint16_t* post, int n);
 const char* zh_warp_name(int index);
+// Tiles up to which a stage of a form runs its kernel for few tiles (0: never),
+// `resident` workgroups of the other fitting a compute unit.  Half floats: one
+// tile per compute unit (8 layers 611x332, 210 tiles: 15.0 us against 15.9; 3
+// layers 1200x700, 874 tiles: 13.5 with the choice against 13.9).  Floats: while
+// the grid is resident as a whole (4 layers 400x300: 7.8 us against 8.7; 8 layers
+// 1200x700, 840 tiles: 32.8 against 34.6).
+uint32_t zh_warp_few_tiles(uint32_t src, uint32_t fmt, uint32_t resident, uint32_t cus);
+// Workgroups of warp kernel `index` that fit a compute unit.
+uint32_t zh_warp_resident(int index, int staged);
 // Does warp kernel `index` have an LDS-staged form (separable, one source)?
 int zh_warp_has_staged(int index);
 // The form of warp kernel `index` (source form, format, mat3 flag and post

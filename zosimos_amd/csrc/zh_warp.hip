@@ -18,10 +18,7 @@ __global__ __launch_bounds__(kBlock, min_waves<V>()) void k_warp(const StageDesc
   warp_stage<V>(dd, run);
 }
 
-// Stages of at most one tile per compute unit: one wave a SIMD, so every
-// instruction's latency shows, and border tests are cheaper than a choice of
-// path (8 layers 611x332, 210 tiles: 15.0 us against 15.9; 3 layers 1200x700,
-// 874 tiles: 13.5 with the choice against 13.9).
+// Stages of few tiles (zh_warp_few_tiles): the kernel without a choice of path.
 template <class V>
 __global__ __launch_bounds__(kBlock) void k_warp_few(const StageDesc* dd, uint32_t run) {
   warp_stage<V, false>(dd, run);
@@ -43,6 +40,11 @@ __global__ __launch_bounds__(kBlock) void k_warp_staged_batch(const BatchDesc* b
   warp_staged_batch<V>(bb);
 }
 
+template <class V>
+constexpr void (*few_fn())(const StageDesc*, uint32_t) {
+  if constexpr (warp_has_few(V::SRC, V::F)) return k_warp_few<V>;
+  else return nullptr;
+}
 template <class V>
 constexpr void (*staged_fn())(const StageDesc*, uint32_t) {
   if constexpr (V::SEP && V::SRC == WSRC_ONE) return k_warp_staged<V>;
@@ -76,7 +78,7 @@ struct WarpEntry {
   const uint16_t* post;
   int n;
   void (*fn)(const StageDesc*, uint32_t);
-  void (*few)(const StageDesc*, uint32_t);
+  void (*few)(const StageDesc*, uint32_t);     // null: no such form
   void (*batch)(const BatchDesc*, uint32_t);
   void (*staged)(const StageDesc*, uint32_t);  // separable one-source forms: LDS-staged tiles
   void (*staged_batch)(const BatchDesc*, uint32_t);
@@ -84,9 +86,9 @@ struct WarpEntry {
 
 #define ZH_WARP_ENTRY(name, src, f, mat, ...)                                                          \
   {#name, src, f, mat, WP_##name, (int)(sizeof(WP_##name) / sizeof(uint16_t)), k_warp<V_##name>,         \
-   k_warp_few<V_##name>, k_warp_batch<V_##name>, nullptr, nullptr},                                                            \
+   few_fn<V_##name>(), k_warp_batch<V_##name>, nullptr, nullptr},                                         \
   {#name "_sep", src, f, mat, WP_##name, (int)(sizeof(WP_##name) / sizeof(uint16_t)), k_warp<VS_##name>, \
-   k_warp_few<VS_##name>, k_warp_batch<VS_##name>, staged_fn<VS_##name>(), staged_batch_fn<VS_##name>()},
+   few_fn<VS_##name>(), k_warp_batch<VS_##name>, staged_fn<VS_##name>(), staged_batch_fn<VS_##name>()},
 static const WarpEntry kWarps[] = {ZH_WARP_LIST(ZH_WARP_ENTRY)};
 #undef ZH_WARP_ENTRY
 
@@ -148,17 +150,28 @@ void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_
   *blocks = (tiles + *run - 1) / *run;
 }
 
-hipError_t zh_launch_warp(int index, int staged, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
-                          uint32_t per_cu, hipStream_t stream) {
-  if (index < 0 || index >= zh::spec::kNumWarps) return hipErrorInvalidValue;
+uint32_t zh_warp_few_tiles(uint32_t src, uint32_t fmt, uint32_t resident, uint32_t cus) {
+  if (!zh::warp_has_few(src, fmt)) return 0;
+  return fmt == zh::FMT_F32 ? resident * cus : cus;
+}
+
+uint32_t zh_warp_resident(int index, int staged) {
+  if (index < 0 || index >= zh::spec::kNumWarps) return 0;
   const auto& e = zh::spec::kWarps[index];
-  if (staged && !e.staged) return hipErrorInvalidValue;
-  const auto fn = staged ? e.staged : tiles <= cus ? e.few : e.fn;
   static uint32_t resident[2][zh::spec::kNumWarps] = {};
   uint32_t& res = resident[staged ? 1 : 0][index];
   if (!res) res = zh::resident_blocks((const void*)(staged ? e.staged : e.fn), 1);
+  return res;
+}
+
+hipError_t zh_launch_warp(int index, int staged, int few, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
+                          uint32_t per_cu, hipStream_t stream) {
+  if (index < 0 || index >= zh::spec::kNumWarps) return hipErrorInvalidValue;
+  const auto& e = zh::spec::kWarps[index];
+  const auto fn = staged ? e.staged : few ? e.few : e.fn;
+  if (!fn) return hipErrorInvalidValue;
   uint32_t blocks, run;
-  zh_warp_grid(tiles, res, cus, per_cu, staged, &blocks, &run);
+  zh_warp_grid(tiles, zh_warp_resident(index, staged), cus, per_cu, staged, &blocks, &run);
   if (blocks == 0) return hipSuccess;
   hipLaunchKernelGGL(fn, dim3(blocks), dim3(zh::kBlock), 0, stream, d_dev, run);
   return hipGetLastError();
