@@ -126,15 +126,17 @@ int zh_warp_has_staged(int index) {
   return index >= 0 && index < zh::spec::kNumWarps && zh::spec::kWarps[index].staged != nullptr;
 }
 
-// Grid of a warp launch over `tiles` tiles, `resident` workgroups fitting the
-// device: blocks of run tiles for the dispatcher to balance (per_cu 0), or a
-// persistent grid (run 0; the staged kernels' pipelined loop, per_cu
-// workgroups per compute unit, which keeps more of each one's taps in the L1,
-// and grids that are resident as a whole, where nothing is left to balance:
-// two 640x480 layers rotated, 300 tiles, 6.65 us against 7.67 in runs).
+// Grid of a warp launch over `tiles` tiles, `resident` workgroups fitting a
+// compute unit: blocks of run tiles for the dispatcher to balance (per_cu 0), or
+// a persistent grid (run 0): the staged kernels' pipelined loop; per_cu
+// workgroups per compute unit, which keeps more of each one's taps in the L1;
+// grids that are resident as a whole, where nothing is left to balance (two
+// 640x480 layers rotated, 300 tiles, 6.65 us against 7.67 in runs); and forms of
+// at most 2 waves a SIMD, whose shares end together (two RGBA32F sources at
+// 3840x2160: 87.3 us, in runs 91.2).
 void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int staged, uint32_t* blocks,
                   uint32_t* run) {
-  if (per_cu || staged || tiles <= resident * cus) {
+  if (per_cu || staged || resident <= 2 || tiles <= resident * cus) {
     *run = 0;
     *blocks = std::min(tiles, (per_cu ? std::min(per_cu, resident) : resident) * cus);
     return;
