@@ -454,7 +454,10 @@ __device__ __forceinline__ void code_group(const Dst& s, Px& X, Codes& c) {
   for (int i = 0; i < kPix; ++i) X[i] = make_float4(clamp01(X[i].x), clamp01(X[i].y), clamp01(X[i].z), clamp01(X[i].w));
 #define ZH_MUX(B)                                                            \
   case B:                                                                    \
-    _Pragma("unroll") for (int i = 0; i < kPix; ++i) c.lo[i] = mux(X[i], B); \
+    _Pragma("unroll") for (int i = 0; i < kPix; ++i) {                       \
+      c.lo[i] = mux(X[i], B);                                                \
+      c.hi[i] = 0u;                                                          \
+    }                                                                        \
     break;
   if constexpr (WIDE) {
     switch (s.bits) {  // uniform

@@ -2,9 +2,9 @@
 // row pitch: conversions (with or without a 3x3 matrix) and the 'over' of two
 // images.  Formats within a class of slots are uniform arguments (zh_any.h),
 // so no compile and no registration stands between a format pair and its
-// kernel.  They stream: measured (and on the interpreter they replace) 26.7 us
-// (220) for 10-bit Bt.2020 to RGBA16F and 33.7 us (139) for RGBA16F to 16-bit
-// sRGB at 3840x2160, 3.7 and 3.9 TB/s; 13.8 us (64) for the 'over' of two
+// kernel.  They stream: measured (and on the interpreter they replace) 26.6 us
+// (221) for 10-bit Bt.2020 to RGBA16F and 29.9 us (139) for RGBA16F to 16-bit
+// sRGB at 3840x2160, 3.7 and 4.4 TB/s; 13.5 us (64) for the 'over' of two
 // 1919x1079 RGBA8 images with padded rows, of which some 6 us are the launch
 // and the tables.
 #include <hip/hip_runtime.h>
