@@ -33,7 +33,7 @@ SOURCES = [
     "zh_dynamic.cpp",
     "zh_jit.cpp",
 ]
-HEADERS = ["zh_stage.h", "zh_codec.h", "zh_device.h", "zh_any.h", "zh_field.h", "zh_spec.h", "zh_prog.h", "zh_spec_kernels.h",
+HEADERS = ["zh_stage.h", "zh_codec.h", "zh_device.h", "zh_divide.h", "zh_any.h", "zh_field.h", "zh_spec.h", "zh_prog.h", "zh_spec_kernels.h",
            "zh_warp_kernels.h", "zh_internal.h",
            "zh_mlp.h"]
 ARCH = "gfx950"

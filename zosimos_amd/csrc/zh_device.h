@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "zh_divide.h"
 #include "zh_codec.h"
 #include "zh_stage.h"
 
@@ -121,19 +122,10 @@ __device__ __forceinline__ float cbrt_s(float x) { return copysignf(pow_pos(fabs
 // SrLab2's cone non-linearity and its inverse (srlab2.frag:87-120).  The
 // shader's pow of a negative base is undefined; below -216/24389 the cube
 // root is taken with its sign.
-//
-// x / c for a constant c in 3 instructions for the general division's 11: the
-// product with 1/c, corrected by its exact remainder (Markstein).  Compared
-// over every float x, this is the rounded quotient for c = 24389, for 2700
-// where |x| > 4.8e-38 (a unit of 1.4e-45 off below) and for 1.16 where |x| >
-// 6.2e-32; v + 0.16 with |v| >= 0.08 is 0 or at least 7e-9.  Infinite x gives
-// NaN, so the last division takes the hardware's fix-up.
-__device__ __forceinline__ float div_const(float x, float c, float rc) {
-  const float q = x * rc;
-  return fmaf(fmaf(-q, c, x), rc, q);
-}
+// The divisions are zh_divide.h's; v + 0.16 with |v| >= 0.08 is 0 or at least 7e-9,
+// and the last one takes the hardware's fix-up for an infinite v.
 __device__ __forceinline__ float srlab_nl(float v) {
-  return fabsf(v) < 216.0f / 24389.0f ? div_const(v * 24389.0f, 2700.0f, 1.0f / 2700.0f)
+  return fabsf(v) < 216.0f / 24389.0f ? div_2700(v * 24389.0f)
                                       : fmaf(1.16f, cbrt_s(v), -0.16f);
 }
 __device__ __forceinline__ float srlab_nl_inv(float v) {
