@@ -36,6 +36,19 @@ def test_registered_and_unsupported_chains():
     assert "jit#" not in text
 
 
+def test_tag_names_the_kernel_that_runs():
+    """An unregistered conversion of in-line formats without run-time kernels
+    runs on the any-format kernel, not the interpreter."""
+    src = z.Descriptor.rgba32f_linear(33, 7)
+    cmd = z.CommandBuffer()
+    a = cmd.input(src)
+    cmd.output(cmd.color_convert(a, z.Color(primaries=z.Primaries.DisplayP3),
+                                 z.Texel(z.SampleBits.UInt8x4, z.SampleParts.BgrA)))
+    assert "[kernel jit#" in describe(cmd)
+    text = describe(cmd, z.PLAN_NO_JIT)
+    assert "[any-format kernel]" in text and "interp" not in text, text
+
+
 def test_unregistered_warp_form_is_compiled_at_run_time():
     d = z.Descriptor(200, 120, W.RGBA16F, W.P3_LINEAR)
     cmd = z.CommandBuffer()

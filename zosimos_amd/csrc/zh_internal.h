@@ -139,6 +139,11 @@ struct Plan {
   std::string text;
 };
 
+// Kernel of a pointwise stage (zh_program::variant): `jit` its run-time kernel
+// is loaded, `aligned` every image is 16-byte aligned, `natural` aligned to its
+// texels; and the tag that names the kernel of aligned images.
+int pointwise_variant(const StagePlan& sp, bool jit, bool aligned, bool natural);
+std::string pointwise_tag(const StagePlan& sp);
 // Does warp stage d get the LDS-staged kernel on tw x th tiles: a separable
 // one-layer one-source form that has one, every tile's source box within
 // kBoxTexels?

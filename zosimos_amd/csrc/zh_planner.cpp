@@ -1229,6 +1229,25 @@ static int any_shape(StageDesc& d, bool flat) {
   return (int)(shape | c << 6);
 }
 
+int pointwise_variant(const StagePlan& sp, bool jit, bool aligned, bool natural) {
+  if (aligned && sp.spec >= 0) return 2;
+  if (aligned && jit) return 6;
+  if (natural && sp.any >= 0) return 7;
+  if (natural && sp.field >= 0) return 8;
+  return aligned && sp.fast ? 1 : 0;
+}
+
+std::string pointwise_tag(const StagePlan& sp) {
+  switch (pointwise_variant(sp, sp.jit >= 0, true, true)) {
+    case 2: return std::string(" [kernel ") + zh_spec_name(sp.spec) + "]";
+    case 6: return " [kernel jit#" + std::to_string(sp.jit) + "]";
+    case 7: return " [any-format kernel]";
+    case 8: return " [field kernel]";
+    case 1: return " [kernel interp-inline]";
+    default: return "";
+  }
+}
+
 bool warp_staged_fits(const StageDesc& d, uint32_t tw, uint32_t th) {
   if (d.kind != STAGE_RESAMPLE || d.variant < 0 || !(d.variant & 1) || d.n_layers != 1) return false;
   const bool has = d.variant >= kJitWarpBase ? jit_warp_has_staged((d.variant - kJitWarpBase) / 2)
@@ -1639,17 +1658,7 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
       std::ostringstream t;
       t << "pointwise " << n.w << "x" << n.h << (flat ? " flat" : "") << ": "
         << describe_code(sp.desc, 0, sp.desc.n_instr);
-      if (sp.spec >= 0)
-        t << " [kernel " << zh_spec_name(sp.spec) << "]";
-      else if (sp.jit >= 0)
-        t << " [kernel jit#" << sp.jit << "]";
-      else if (sp.fast)
-        t << " [kernel interp-inline]";
-      else if (sp.any >= 0)
-        t << " [any-format kernel]";
-      else if (sp.field >= 0)
-        t << " [field kernel]";
-      sp.text = t.str();
+      sp.text = t.str() + pointwise_tag(sp);
       plan.stages.push_back(sp);
       continue;
     }

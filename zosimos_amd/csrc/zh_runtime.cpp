@@ -645,10 +645,10 @@ static zh_status alloc_device(zh_program* p) {
         p->jit_batch_resident[s] = (uint32_t)n;
       p->jit_stage_fn[s] = f;
       p->jit_few_fn[s] = ff;
+      p->jit_batch_fn[s] = fb;
       WarpForm form;
       if (ff && warp_form_of(sp.desc.variant, &form))
         p->few_tiles[s] = zh_warp_few_tiles(form.src, form.fmt, p->jit_resident[s], (uint32_t)ctx->cus);
-      p->jit_batch_fn[s] = fb;
       continue;
     }
     if (sp.desc.kind == STAGE_RESAMPLE && sp.desc.variant >= 0 && !sp.staged) {
@@ -663,7 +663,7 @@ static zh_status alloc_device(zh_program* p) {
     if (p->arena || jit_kernels(sp.jit, ctx->device, &f, &fb, &why) != ZH_OK) {
       sp.jit = -1;
       if (k != std::string::npos)
-        sp.text = sp.text.substr(0, k) + " [kernel interp-inline]" +
+        sp.text = sp.text.substr(0, k) + pointwise_tag(sp) +
                   (p->arena ? std::string() : " (run-time kernel unavailable: " + why.substr(0, 120) + ")");
       continue;
     }
@@ -1137,8 +1137,7 @@ static zh_status bind(zh_program* p, const zh_binding* b, uint32_t n) {
           const uint32_t bpp = d.slot[k].bpp, align = bpp == 1 || bpp == 3 ? 1u : bpp == 2 || bpp == 6 ? 2u : 4u;
           natural = natural && d.slot[k].ptr % align == 0 && (d.flat || d.slot[k].row_stride % align == 0);
         }
-        variant[s] = aligned && sp.spec >= 0 ? 2 : aligned && jit ? 6 : natural && sp.any >= 0 ? 7
-                     : natural && sp.field >= 0 ? 8 : aligned && sp.fast ? 1 : 0;
+        variant[s] = pointwise_variant(sp, jit, aligned, natural);
       }
     }
     p->h_stages[s] = d;
