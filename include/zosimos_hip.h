@@ -311,6 +311,9 @@ typedef struct zh_op {
  * instead of two tile queues one after the other.  Measured slower on
  * MI355X, so not the default. */
 #define ZH_PLAN_PAIR 16u
+/* Run every pointwise and resample stage on the general interpreter, none on
+ * a specialised kernel: the path those are compared with. */
+#define ZH_PLAN_INTERPRETER 32u
 
 /* Lower a High program (Program::lower_to, program.rs:1304).  `textures`
  * holds the descriptor of every texture id.  `ctx` may be NULL: the plan is

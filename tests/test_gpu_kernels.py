@@ -2,13 +2,14 @@
 general interpreter on the same program.
 
 Each case is a one-stage program whose micro-op sequence matches one
-registered signature.  It runs three ways: as planned (the specialised
-kernel: flat, 16-byte aligned images), with padded rows (a different
-descriptor, so the planner falls back to the 2-D interpreter), and -- for the
-4- and 8-byte formats -- with the same executable bound to images at an
-address that is not 16-byte aligned (the runtime then launches the
-interpreter and captures its graph again).  Sizes leave a partial group of
-pixels at the end of the image.
+registered signature.  Planned, it runs on the specialised kernel (flat,
+16-byte aligned images); on the any-format kernel, where it has one of its
+shapes, or the interpreter with the same executable bound to images at an
+address that is not 16-byte aligned (4- and 8-byte formats; the runtime
+captures its graph again) and with padded rows (a different descriptor, planned
+in 2-D).  Lowered for the interpreter (ZH_PLAN_INTERPRETER) it runs all three
+ways again: with in-line codecs, with the general codecs, and in 2-D.  Sizes
+leave a partial group of pixels at the end of the image.
 
 Bars: 8-bit outputs within 1 code of the FP64 oracle (colour where the 8-bit
 alpha is non-zero after 'over'); f16 outputs within 1 ulp or 1e-6 absolute;
@@ -192,9 +193,13 @@ def test_specialised_kernel_matches_oracle(ctx, name, w, h):
     got = launch(ctx, exe, imgs, o, od)
     check(f"{name}_{w}x{h}_spec", got, want, out_kind, w, h, mask)
 
-    # Same executable, images at an address that is not 16-byte aligned: the
-    # interpreter runs (the graph is captured again), then the aligned images
-    # once more.
+    plain = z.Linker.from_included().compile(cmd).lower_to(ctx, z.PLAN_INTERPRETER)
+    assert "[kernel interp-inline]" in plain.describe()
+    check(f"{name}_{w}x{h}_interp_inline", launch(ctx, plain, imgs, o, od), want, out_kind, w, h, mask)
+
+    # The same executables, images at an address that is not 16-byte aligned:
+    # the any-format kernel or the interpreter runs (the graph is captured
+    # again), then the aligned images once more.
     bpp = {"s8": 4, "l8": 4, "h": 8, "lab": 8, "f": 16}
     if all(bpp[k] < 16 for k in kinds + [out_kind]):
         keep, mis = [], {}
@@ -206,24 +211,30 @@ def test_specialised_kernel_matches_oracle(ctx, name, w, h):
             mis[r] = img
         big_o = ctx.image(z.Descriptor.rgba8_srgb(w * h * bpp[out_kind] // 4 + 4, 1))
         out = ctx.wrap(od, big_o.device_ptr + bpp[out_kind], w * h * bpp[out_kind])
-        exe.launch(mis, {o: out})
-        ctx.sync()
-        check(f"{name}_{w}x{h}_unaligned", out.download().reshape(-1), want, out_kind, w, h, mask)
+        for tag, e in (("unaligned", exe), ("interp_unaligned", plain)):
+            out.upload(np.zeros(w * h * bpp[out_kind], np.uint8))
+            e.launch(mis, {o: out})
+            ctx.sync()
+            check(f"{name}_{w}x{h}_{tag}", out.download().reshape(-1), want, out_kind, w, h, mask)
         got2 = launch(ctx, exe, imgs, o, od)
         assert np.array_equal(got2, got)
         for img in list(mis.values()) + [out]:
             img.free()
         del keep, big_o
 
-    # Padded rows: the planner takes the 2-D interpreter.
+    # Padded rows: the planner takes the 2-D form of the any-format kernel, or
+    # the interpreter for the chains that are none of its shapes.
     cmd, ins, o, od = build_case(name, w, h, row_pad=16)
-    exe = z.Linker.from_included().compile(cmd).lower_to(ctx)
-    assert "[kernel" not in exe.describe()
+    prog = z.Linker.from_included().compile(cmd)
     imgs = {}
     for (r, d), raw in zip(ins.items(), host):
         imgs[r] = ctx.image(d)
         imgs[r].upload(raw)
-    check(f"{name}_{w}x{h}_interp", launch(ctx, exe, imgs, o, od), want, out_kind, w, h, mask)
+    for tag, flags in (("padded", 0), ("interp_padded", z.PLAN_INTERPRETER)):
+        exe = prog.lower_to(ctx, flags)
+        text = exe.describe()
+        assert "[kernel" not in text and ("[any-format kernel]" in text) == (not flags and "oklab" not in name), text
+        check(f"{name}_{w}x{h}_{tag}", launch(ctx, exe, imgs, o, od), want, out_kind, w, h, mask)
 
 
 def test_c2_kernel_multi_step_grid(ctx):

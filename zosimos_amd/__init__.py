@@ -696,6 +696,7 @@ PLAN_NO_GRAPH = 2
 PLAN_NO_JIT = 4
 PLAN_STAGED = 8
 PLAN_PAIR = 16
+PLAN_INTERPRETER = 32
 
 
 class Program:

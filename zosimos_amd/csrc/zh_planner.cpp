@@ -1314,6 +1314,7 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
   if (st != ZH_OK) return st;
   if (outputs.empty()) return fail(ZH_ERR_INVALID_ARGUMENT, "program has no output");
   const bool strict = (flags & ZH_PLAN_STRICT_REGISTERS) != 0;
+  const bool interpreter = (flags & ZH_PLAN_INTERPRETER) != 0;
 
   // Uses reachable from the outputs.
   std::vector<bool> live(B.nodes.size(), false);
@@ -1612,7 +1613,7 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
       sp.fast = fast;
       // A registered signature runs as a specialised kernel (zh_spec.h).
       sp.spec = -1;
-      if (fast) {
+      if (fast && !interpreter) {
         uint16_t sig[kMaxInstr];
         for (uint32_t i = 0; i < sp.desc.n_instr; ++i) {
           const Instr& in = sp.desc.code[i];
@@ -1645,8 +1646,10 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
           s.row_stride = (uint64_t)s.width * s.bpp;
         }
       }
-      sp.any = any_shape(sp.desc, flat);
-      if (!flat && sp.any < 0) sp.field = field_shape(sp.desc);
+      if (!interpreter) {
+        sp.any = any_shape(sp.desc, flat);
+        if (!flat && sp.any < 0) sp.field = field_shape(sp.desc);
+      }
       for (size_t k = 0; k < sp.slot_ref.size(); ++k)
         if (sp.slot_ref[k] > -1000000 || sp.slot_ref[k] < -2000000000ll) {
           // quantisation-only slots (strict mode) carry no traffic
@@ -1823,8 +1826,8 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
     // A registered affine layer form runs as a warp kernel (zh_warp.hip) on
     // 64 x 16 tiles; the interpreter kernels stay valid on the same tiles as
     // the fallback for images the warp kernel cannot address.
-    sp.desc.variant = bil ? warp_variant(sp.desc, flags) : -1;
-    if (!bil) sp.move = move_words(sp.desc);
+    sp.desc.variant = bil && !interpreter ? warp_variant(sp.desc, flags) : -1;
+    if (!bil && !interpreter) sp.move = move_words(sp.desc);
     if (sp.desc.variant >= 0) {
       max_box = 0;
       choose_tiles({{64, 16}});
