@@ -1,5 +1,6 @@
 """Helpers of the GPU parity tests: run a program through the C ABI and
 compare with the FP64 oracle."""
+import re
 import sys
 
 import numpy as np
@@ -21,6 +22,19 @@ def run(ctx, commands, inputs, host, outputs, flags=0, launches=1):
         exe.launch(imgs_in, imgs_out)
     ctx.sync()
     return {reg: img.download() for reg, img in imgs_out.items()}, exe
+
+
+def run_both(ctx, commands, inputs, host, outputs):
+    """run(), and the same program on the interpreter: the any-format, field and
+    move kernels give the interpreter's bytes."""
+    out, exe = run(ctx, commands, inputs, host, outputs)
+    ref, plain = run(ctx, commands, inputs, host, outputs, flags=z.PLAN_INTERPRETER)
+    assert not re.search(r"kernel\]|\[kernel (?!interp-inline)", plain.describe()), plain.describe()
+    stages = [line for line in exe.describe().splitlines() if line.startswith("stage ")]
+    if all(re.search(r"\[(any-format|field|move) kernel\]", line) for line in stages):
+        for o in outputs:
+            assert np.array_equal(out[o], ref[o]), exe.describe()
+    return out, exe
 
 
 def report(name, **kv):

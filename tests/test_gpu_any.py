@@ -8,7 +8,7 @@ import zosimos_amd as z
 from oracle import color as C
 from oracle import stage as S
 
-from gpu_util import report, run
+from gpu_util import report, run_both
 
 pytestmark = pytest.mark.gpu
 
@@ -43,23 +43,31 @@ def _decoded(bits, parts, transfer, raw, codes):
     return S.stage_decode(codes, bits, parts, transfer)
 
 
+def _pitch(w, bpp, pad):
+    """Row bytes: a multiple of 4 for a positive pad, and for a negative one the
+    odd number of texels that leaves rows of 1-, 2-, 3- and 6-byte texels at
+    every address their size allows."""
+    return 0 if not pad else (w * bpp + pad + 3) // 4 * 4 if pad > 0 else (w | 1) * bpp - 2 * pad * bpp
+
+
 # Rows of 1-9 texels (partial groups only, one whole group, a whole and a
 # partial one), a row past one workgroup, and a padded pitch.
-@pytest.mark.parametrize("w,h,pad", [(1, 1, 0), (3, 5, 0), (4, 2, 12), (7, 3, 4), (9, 1, 0), (1031, 2, 0), (1029, 3, 20)])
+@pytest.mark.parametrize("w,h,pad", [(1, 1, 0), (3, 5, 0), (4, 2, 12), (7, 3, 4), (9, 1, 0), (1031, 2, 0), (1029, 3, 20),
+                                     (7, 5, -1), (1024, 5, -1), (1027, 3, -2)])
 @pytest.mark.parametrize("bits,parts,transfer", FORMATS)
 def test_any_format_conversion(ctx, bits, parts, transfer, w, h, pad):
     """Decode to RGBA32F (2-D for a padded pitch, flat otherwise), then encode
-    the decoded values back: bit-exact for linear transfers; a transfer is
+    the decoded values back (both the interpreter's bytes): bit-exact for linear transfers; a transfer is
     compared within the accuracy of two pow implementations (a few f32 ulps
     through an exponent of at most 2.4: 4e-6 relative, 1e-6 absolute)."""
     bpp = z.BITS_BYTES[bits]
     raw, codes = _texels(bits, w * h, [bits, parts, w, h])
-    pitch = (w * bpp + pad + 3) // 4 * 4 if pad else 0
+    pitch = _pitch(w, bpp, pad)
     src = z.Descriptor(w, h, z.Texel(bits, parts), z.Color(transfer=transfer), pitch)
     cmd = z.CommandBuffer()
     a = cmd.input(src)
     o, od = cmd.output(cmd.color_convert(a, LINEAR, F32))
-    out, exe = run(ctx, cmd, {a: src}, {a: raw.reshape(h, w * bpp)}, {o: od})
+    out, exe = run_both(ctx, cmd, {a: src}, {a: raw.reshape(h, w * bpp)}, {o: od})
     assert "any-format kernel" in exe.describe()
     got = out[o].view(np.float32).reshape(-1, 4)
     want = _decoded(bits, parts, transfer, raw, codes)
@@ -67,13 +75,16 @@ def test_any_format_conversion(ctx, bits, parts, transfer, w, h, pad):
         assert np.array_equal(got, want.astype(np.float32))
     else:
         assert np.all(np.abs(got - want) <= 4e-6 * np.abs(want) + 1e-6)
-    if bits in (SB.UInt16x3, SB.UInt16x4) or transfer != T.Linear:
-        return
+    # Padded rows here too: the stores of the tight output then start at every
+    # address a row of its texels can.
     cmd = z.CommandBuffer()
-    f32 = z.Descriptor(w, h, F32, LINEAR)
+    f32 = z.Descriptor(w, h, F32, LINEAR, w * 16 + 16 if pad else 0)
     a = cmd.input(f32)
     o, od = cmd.output(cmd.color_convert(a, src.color, src.texel))
-    out, _ = run(ctx, cmd, {a: f32}, {a: got.view(np.uint8).reshape(h, w * 16)}, {o: od})
+    out, exe = run_both(ctx, cmd, {a: f32}, {a: got.view(np.uint8).reshape(h, w * 16)}, {o: od})
+    assert "any-format kernel" in exe.describe()
+    if bits in (SB.UInt16x3, SB.UInt16x4) or transfer != T.Linear:
+        return
     pad4 = np.zeros((w * h, 4), np.uint8)
     pad4[:, :bpp] = out[o].reshape(w * h, bpp)
     mask = np.uint32(0xffffffff) if bpp >= 4 else np.uint32((1 << (8 * bpp)) - 1)
@@ -112,9 +123,10 @@ def test_any_format_over(ctx, below, above, w, h, pad):
         fa, fb = cmd.color_convert(a, LINEAR, lin), cmd.color_convert(b, LINEAR, lin)
         v = cmd.blend(fa, z.Rectangle(0, 0, w, h), fb)
         o, od = cmd.output(cmd.color_convert(v, z.Color(primaries=primaries, transfer=T.Linear), lin))
-        out, exe = run(ctx, cmd, {a: da, b: db}, {a: ra, b: rb}, {o: od})
-        if below != above or below == "u16" or pad:
-            assert "[kernel" in exe.describe() or "any-format kernel" in exe.describe()
+        out, exe = run_both(ctx, cmd, {a: da, b: db}, {a: ra, b: rb}, {o: od})
+        # Tight images of in-line formats have a registered or compiled kernel.
+        tag = "[any-format kernel]" if pad or below == "u16" else "[kernel "
+        assert tag in exe.describe() and "interp" not in exe.describe()
         want = C.unpremultiply(C.over(C.premultiply(vb), C.premultiply(va)))
         if primaries != z.Primaries.Bt709:
             want[..., :3] = want[..., :3] @ C.convert_matrix(3, primaries, 5).T

@@ -1,5 +1,5 @@
 """The filter, noise and lookup kernels (zh_field.hip) at the edges of their
-strips, tiles and caches, against the oracle."""
+strips, tiles and caches, against the oracle and the interpreter's bytes."""
 import numpy as np
 import pytest
 
@@ -7,7 +7,7 @@ import zosimos_amd as z
 from oracle import color as C
 from oracle import pipelines as PL
 
-from gpu_util import run
+from gpu_util import run_both
 
 pytestmark = pytest.mark.gpu
 
@@ -42,7 +42,7 @@ def test_box3_strips(ctx, kind, direction, w, h):
     cmd = z.CommandBuffer()
     a = cmd.input(d)
     o, od = cmd.output(cmd.derivative(a, z.DerivativeMethod.Sobel, direction))
-    out, exe = run(ctx, cmd, {a: d}, {a: raw.view(np.uint8).reshape(h, -1)}, {o: od})
+    out, exe = run_both(ctx, cmd, {a: d}, {a: raw.view(np.uint8).reshape(h, -1)}, {o: od})
     assert "field kernel" in exe.describe()
     want = PL.box3(v, PL.derivative_weights(z.DerivativeMethod.Sobel, width=direction == z.Direction.Width))
     got = out[o].reshape(-1).view(raw.dtype).reshape(h, w, 4)
@@ -57,6 +57,26 @@ def test_box3_strips(ctx, kind, direction, w, h):
         assert np.all(np.abs(got.astype(np.float64) - want) <= 4e-7 + step)
 
 
+@pytest.mark.parametrize("transfer", [T.Bt709, T.Bt470M, T.Bt601, T.Smpte240, T.Bt2020_10bit, T.Smpte2084, T.Srgb])
+@pytest.mark.parametrize("bits", [SB.UInt8x4, SB.UInt16x4])
+def test_box3_transfers(ctx, bits, transfer):
+    """Derivatives of images with a transfer, every 8-bit code among them: the
+    interpreter's bytes (run_both), NaN where it has them (SMPTE 240 has none
+    between its segments, so there no zero weight may be skipped)."""
+    w, h = 70, 37
+    rng = np.random.default_rng(int(transfer))
+    raw = rng.integers(0, 256, (h, w * z.BITS_BYTES[bits]), dtype=np.uint8)
+    raw.reshape(-1)[:256] = np.arange(256)
+    d = z.Descriptor(w, h, z.Texel(bits, SP.RgbA), z.Color(transfer=transfer))
+    for method in (z.DerivativeMethod.Sobel, z.DerivativeMethod.Scharr3):
+        cmd = z.CommandBuffer()
+        a = cmd.input(d)
+        v = cmd.derivative(a, method, z.Direction.Width)
+        o, od = cmd.output(v)
+        _, exe = run_both(ctx, cmd, {a: d}, {a: raw}, {o: od})
+        assert "field kernel" in exe.describe()
+
+
 # Octaves past the cached ones, cells smaller than a pixel (nothing fits the
 # cache, or only the low octaves), several tiles with ragged edges, an
 # octave count of 0.
@@ -68,7 +88,7 @@ def test_noise_cache(ctx, w, h, octaves, scale):
     n = z.FractalNoise(octaves, 0.25, 0.75, scale)
     cmd = z.CommandBuffer()
     o, od = cmd.output(cmd.distribution_fractal_noise(z.Descriptor.rgba32f_linear(w, h), n))
-    out, exe = run(ctx, cmd, {}, {}, {o: od})
+    out, exe = run_both(ctx, cmd, {}, {}, {o: od})
     assert "field kernel" in exe.describe()
     want = PL.fractal_noise(w, h, octaves, n.initial_amplitude, n.amplitude_damping, scale).astype(np.float32)
     assert np.array_equal(out[o].view(np.float32).reshape(h, w, 4), want)
@@ -84,7 +104,7 @@ def test_lookup(ctx, kind, ow, oh):
     cmd = z.CommandBuffer()
     a = cmd.input(d)
     o, od = cmd.output(cmd.resize(a, ow, oh))
-    out, exe = run(ctx, cmd, {a: d}, {a: raw.view(np.uint8).reshape(h, -1)}, {o: od})
+    out, exe = run_both(ctx, cmd, {a: d}, {a: raw.view(np.uint8).reshape(h, -1)}, {o: od})
     assert "field kernel" in exe.describe()
     f = np.float32
     ramp = np.zeros((oh, ow, 4), f)
@@ -104,7 +124,7 @@ def test_generator_rows_at_any_address(ctx, bits, parts, w, h):
     d = z.Descriptor(w, h, z.Texel(bits, parts), LINEAR)
     cmd = z.CommandBuffer()
     o, od = cmd.output(cmd.bilinear(d, z.Bilinear(u_max=(1.0, 0.0, 1.0, 1.0), v_max=(0.0, 1.0, 0.0, 0.0))))
-    out, exe = run(ctx, cmd, {}, {}, {o: od})
+    out, exe = run_both(ctx, cmd, {}, {}, {o: od})
     assert "field kernel" in exe.describe()
     f = np.float32
     u = np.broadcast_to(((np.arange(w, dtype=f) + f(0.5)) / f(w))[None, :], (h, w))

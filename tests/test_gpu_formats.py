@@ -1,6 +1,8 @@
 """GPU parity of the texel codecs that the workloads do not exercise: the
 non-sRGB transfer functions, native BGRA8, the wide 16-bit layouts and the
-rarer packed layouts of stage.frag.  Every call goes through the C ABI.
+rarer packed layouts of stage.frag.  Every call goes through the C ABI, and
+runs on the planned kernel and on the interpreter (run_both): where the planned
+one is the any-format kernel, both give the same bytes.
 
 Bars:
 - packed layouts with a linear transfer: decode bit-exact against the FP32
@@ -24,7 +26,7 @@ import zosimos_amd as z
 from oracle import color as C
 from oracle import stage as S
 
-from gpu_util import report, run
+from gpu_util import report, run_both
 
 pytestmark = pytest.mark.gpu
 
@@ -56,7 +58,7 @@ def decode_on_gpu(ctx, codes, bits, parts, transfer, w=256):
     cmd = z.CommandBuffer()
     a = cmd.input(src)
     o, od = cmd.output(cmd.color_convert(a, z.Color(transfer=T.Linear), F32))
-    out, _ = run(ctx, cmd, {a: src}, {a: _raw(codes, bpp, w)}, {o: od})
+    out, _ = run_both(ctx, cmd, {a: src}, {a: _raw(codes, bpp, w)}, {o: od})
     return out[o].view(np.float32).reshape(-1, 4)
 
 
@@ -70,7 +72,7 @@ def encode_on_gpu(ctx, values, bits, parts, transfer, w=256):
     cmd = z.CommandBuffer()
     a = cmd.input(f32)
     o, _ = cmd.output(cmd.color_convert(a, dst.color, dst.texel))
-    out, _ = run(ctx, cmd, {a: f32}, {a: np.ascontiguousarray(values, np.float32).view(np.uint8).reshape(h, w * 16)},
+    out, _ = run_both(ctx, cmd, {a: f32}, {a: np.ascontiguousarray(values, np.float32).view(np.uint8).reshape(h, w * 16)},
                  {o: dst})
     raw = out[o].reshape(n, bpp)
     pad = np.zeros((n, 4), np.uint8)
@@ -118,7 +120,7 @@ def test_wide_16bit_layouts_round_trip(ctx, bits, parts):
     cmd = z.CommandBuffer()
     a = cmd.input(src)
     o, od = cmd.output(cmd.color_convert(a, z.Color(transfer=T.Linear), F32))
-    out, _ = run(ctx, cmd, {a: src}, {a: raw}, {o: od})
+    out, _ = run_both(ctx, cmd, {a: src}, {a: raw}, {o: od})
     got = out[o].view(np.float32).reshape(-1, 4)
     want = vals.astype(np.float32) / np.float32(65535.0)
     assert np.array_equal(got[:, :ch], want)
@@ -129,14 +131,14 @@ def test_wide_16bit_layouts_round_trip(ctx, bits, parts):
     f32 = _f32_desc(w, h)
     a = cmd.input(f32)
     o, _ = cmd.output(cmd.color_convert(a, src.color, src.texel))
-    out, _ = run(ctx, cmd, {a: f32}, {a: got.view(np.uint8).reshape(h, w * 16)}, {o: src})
+    out, _ = run_both(ctx, cmd, {a: f32}, {a: got.view(np.uint8).reshape(h, w * 16)}, {o: src})
     assert np.array_equal(out[o], raw)
     # truncating encode of arbitrary values, clamped to [0, 1]
     v = rng.uniform(-0.2, 1.2, (w * h, 4)).astype(np.float32)
     cmd = z.CommandBuffer()
     a = cmd.input(f32)
     o, _ = cmd.output(cmd.color_convert(a, src.color, src.texel))
-    out, _ = run(ctx, cmd, {a: f32}, {a: v.view(np.uint8).reshape(h, w * 16)}, {o: src})
+    out, _ = run_both(ctx, cmd, {a: f32}, {a: v.view(np.uint8).reshape(h, w * 16)}, {o: src})
     exp = (np.clip(v, 0, 1) * np.float32(65535.0)).astype(np.uint32).astype(np.uint16)[:, :ch]
     assert np.array_equal(out[o].view(np.uint16).reshape(-1, ch), exp)
 
@@ -267,7 +269,7 @@ def test_native_bgra8_decode_encode(ctx, transfer):
     cmd = z.CommandBuffer()
     a = cmd.input(src)
     o, od = cmd.output(cmd.color_convert(a, z.Color(transfer=T.Linear), F32))
-    out, _ = run(ctx, cmd, {a: src}, {a: raw}, {o: od})
+    out, _ = run_both(ctx, cmd, {a: src}, {a: raw}, {o: od})
     got = out[o].view(np.float32).reshape(h, w, 4)
     bgra = raw.reshape(h, w, 4)
     rgba = bgra[..., [2, 1, 0, 3]]
@@ -289,7 +291,7 @@ def test_native_bgra8_decode_encode(ctx, transfer):
     cmd = z.CommandBuffer()
     a = cmd.input(f32)
     o, _ = cmd.output(cmd.color_convert(a, col, tex))
-    out, _ = run(ctx, cmd, {a: f32}, {a: v.view(np.uint8).reshape(h, w * 16)}, {o: src})
+    out, _ = run_both(ctx, cmd, {a: f32}, {a: v.view(np.uint8).reshape(h, w * 16)}, {o: src})
     gotb = out[o].reshape(h, w, 4)
     if transfer == T.Srgb:
         want_rgb = C.encode_u8(v.astype(np.float64), T.Srgb)[..., :3]
@@ -303,7 +305,7 @@ def test_native_bgra8_decode_encode(ctx, transfer):
     cmd = z.CommandBuffer()
     a = cmd.input(f32)
     o, _ = cmd.output(cmd.color_convert(a, col, tex))
-    out, _ = run(ctx, cmd, {a: f32}, {a: got.view(np.uint8).reshape(h, w * 16)}, {o: src})
+    out, _ = run_both(ctx, cmd, {a: f32}, {a: got.view(np.uint8).reshape(h, w * 16)}, {o: src})
     assert np.array_equal(out[o], raw)
 
 
@@ -317,5 +319,5 @@ def test_bgra8_to_rgba8_is_a_byte_permutation(ctx, transfer):
     cmd = z.CommandBuffer()
     a = cmd.input(src)
     o, _ = cmd.output(cmd.color_convert(a, col, dst.texel))
-    out, _ = run(ctx, cmd, {a: src}, {a: raw}, {o: dst})
+    out, _ = run_both(ctx, cmd, {a: src}, {a: raw}, {o: dst})
     assert np.array_equal(out[o].reshape(h, w, 4), raw.reshape(h, w, 4)[..., [2, 1, 0, 3]])

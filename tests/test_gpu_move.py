@@ -1,5 +1,6 @@
 """The texel-moving nearest kernel (zh_move.hip) at tile edges, for stacked
-and partly outside paints, against a numpy restatement of the FP64 maps."""
+and partly outside paints, against a numpy restatement of the FP64 maps and
+the interpreter's bytes."""
 import math
 
 import numpy as np
@@ -9,7 +10,7 @@ import zosimos_amd as z
 from oracle import pipelines as PL
 from zosimos_amd import workloads as W
 
-from gpu_util import run
+from gpu_util import run_both
 
 pytestmark = pytest.mark.gpu
 
@@ -44,7 +45,7 @@ def test_inscribe_moves_bytes(ctx, kind, w, h, fw, fh, pad):
     b, f, g = cmd.input(db), cmd.input(df), cmd.input(dg)
     v = cmd.inscribe(cmd.inscribe(b, z.Rectangle(0, 0, fw, fh), f), z.Rectangle(0, 0, gw, gh), g)
     o, od = cmd.output(v)
-    out, exe = run(ctx, cmd, {b: db, f: df, g: dg}, {b: _bytes(vb), f: _bytes(vf), g: _bytes(vg)}, {o: od})
+    out, exe = run_both(ctx, cmd, {b: db, f: df, g: dg}, {b: _bytes(vb), f: _bytes(vf), g: _bytes(vg)}, {o: od})
     want = vb.copy()
     # Rectangle::normalize takes max_y = y + width: the quad of a paint is as
     # tall as the rectangle is wide, cut at the target.
@@ -69,7 +70,7 @@ def test_nearest_affine_moves_texels(ctx, kind, degrees, scale):
     cmd = z.CommandBuffer()
     b, f = cmd.input(db), cmd.input(df)
     o, od = cmd.output(cmd.affine(b, aff, f))
-    out, exe = run(ctx, cmd, {b: db, f: df}, {b: _bytes(vb), f: _bytes(vf)}, {o: od})
+    out, exe = run_both(ctx, cmd, {b: db, f: df}, {b: _bytes(vb), f: _bytes(vf)}, {o: od})
     assert "move kernel" in exe.describe()
     got = out[o].reshape(h, w, -1)
     m = np.array(np.float32(aff.transformation), np.float64).reshape(3, 3)
@@ -93,7 +94,7 @@ def test_crop_moves_texels(ctx, w, h, rect):
     cmd = z.CommandBuffer()
     a = cmd.input(d)
     o, od = cmd.output(cmd.crop(a, z.Rectangle(*rect)))
-    out, exe = run(ctx, cmd, {a: d}, {a: _bytes(v)}, {o: od})
+    out, exe = run_both(ctx, cmd, {a: d}, {a: _bytes(v)}, {o: od})
     assert "move kernel" in exe.describe()
     want = PL.crop(v.astype(np.float64), rect)
     assert np.array_equal(out[o].reshape(h, w, 4), want.astype(np.uint8))

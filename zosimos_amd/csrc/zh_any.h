@@ -444,6 +444,7 @@ __device__ __forceinline__ void code_group(const Dst& s, Px& X, Codes& c) {
   if (WIDE && s.bits == 18) {  // uniform
 #pragma unroll
     for (int i = 0; i < kPix; ++i) {
+      round_f32(X[i]);
       c.lo[i] = pack_f16(X[i].x, X[i].y);
       c.hi[i] = pack_f16(X[i].z, X[i].w);
     }
@@ -503,6 +504,7 @@ __device__ __forceinline__ void put_group(const Dst& s, gbyte* q, int n, Px& X, 
   } else if constexpr (D == DST_F16) {
 #pragma unroll
     for (int i = 0; i < kPix; ++i) {
+      round_f32(X[i]);
       c.lo[i] = pack_f16(X[i].x, X[i].y);
       c.hi[i] = pack_f16(X[i].z, X[i].w);
     }

@@ -36,11 +36,6 @@ __device__ __forceinline__ void fetch(const Src& a, const Src& b, Group& g) {
     if (B != SRC_F32 && b.bpp != 16) load_group(texels(b, g), b.bpp, g.n, g.b);
 }
 
-// A matrix row on a colour, contracted as the interpreter's is.
-__device__ __forceinline__ float row3(const float* m, float4 v) {
-  return fmaf(m[2], v.z, fmaf(m[0], v.x, m[1] * v.y));
-}
-
 // The colour of the group under the shape's program.  The arithmetic is the
 // interpreter's, instruction by instruction (zh_kernels.hip run()).
 template <int A, int B, bool POW>

@@ -115,6 +115,18 @@ __device__ __forceinline__ float3 mat3(const __attribute__((address_space(4))) f
                      m[6] * v.x + m[7] * v.y + m[8] * v.z);
 }
 
+// A matrix row on a colour.  The sums are written out: left to the compiler,
+// which product each fma takes differs from kernel to kernel, and with it the
+// last bit.
+__device__ __forceinline__ float row3(const float* m, float4 v) {
+  return fmaf(m[2], v.z, fmaf(m[0], v.x, m[1] * v.y));
+}
+
+// Round v to FP32 before it is rounded to half floats: the compiler otherwise
+// fuses a last fma with the conversion (v_fma_mixlo_f16), which rounds once and
+// differs at ties.
+__device__ __forceinline__ void round_f32(float4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+
 // Signed cube root: sign(x) 2^(log2|x| / 3) through the hardware log2/exp2
 // (relative error ~1e-7 over the colour range; cbrt(0) = 0 since
 // exp2(-inf) = 0).
