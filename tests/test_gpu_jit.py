@@ -38,7 +38,8 @@ def test_unregistered_chain_runs_a_compiled_kernel(ctx):
 
 def test_compiled_kernel_batch_of_ragged_images(ctx):
     """Five images of the signature: one launch of the compiled batch kernel
-    (chunks of 16,384 pixels), each image equal to its interpreter result."""
+    (one chunk of 1,024 pixels after the other; test_gpu_spec_chunks.py has the
+    longer ones), each image within 1 code of its interpreter result."""
     sizes = [(1, 1), (7, 5), (129, 127), (300, 61), (16385, 2)]
     cmd = z.CommandBuffer()
     regs, inputs, host = [], {}, {}
@@ -206,3 +207,62 @@ def test_compiled_form_of_few_tiles(ctx, texel, w, h, few, degrees):
     codes = C.encode_u8(PL.apply3(C.convert_matrix(7, 3, 5), straight), 5)
     mr, ma, _ = compare_u8(f"jitw_few_{texel}_{w}x{h}_{degrees}", out[o], codes, alpha_ok=straight[..., 3] > 0.02)
     assert mr <= 1 and ma <= 1
+
+
+@pytest.mark.parametrize("w,h", [(5, 3), (257, 130)])
+def test_compiled_srlab2_chain(ctx, w, h):
+    """SrLab2 of linear RGBA32F texels into half-float and float Lab (no
+    registered signature): compiled, the interpreter's bytes, and within 2e-5 of
+    the FP64 oracle's L, a, b (f16 targets: half an f16 ulp of values below 2,
+    2^-11, on top)."""
+    from oracle import color as C
+    rng = np.random.default_rng([w, h])
+    v = rng.random((h, w, 4)).astype(np.float32)
+    v.reshape(-1)[:8] = [0, 0, 0, 1, 1, 1, 1, 1]
+    for bits, tol in ((z.SampleBits.Float16x4, 2e-5 + 2.0 ** -11), (z.SampleBits.Float32x4, 2e-5)):
+        d = z.Descriptor.rgba32f_linear(w, h)
+        cmd = z.CommandBuffer()
+        a = cmd.input(d)
+        o, od = cmd.output(cmd.color_convert(a, z.Color.SRLAB2_D65, z.Texel(bits, z.SampleParts.LabA)))
+        host = {a: v.view(np.uint8).reshape(h, -1)}
+        out, exe = run(ctx, cmd, {a: d}, host, {o: od})
+        text = exe.describe()
+        assert "[kernel jit#" in text and "unavailable" not in text, text
+        ref, _ = run(ctx, cmd, {a: d}, host, {o: od}, flags=z.PLAN_INTERPRETER)
+        assert np.array_equal(out[o], ref[o])
+        dt = np.float16 if bits == z.SampleBits.Float16x4 else np.float32
+        got = np.asarray(out[o]).reshape(-1).view(dt).reshape(h, w, 4).astype(np.float64)
+        assert np.abs(got[..., :3] - C.rgb_to_srlab2(v[..., :3])).max() <= tol
+
+
+@pytest.mark.parametrize("source", ["s8", "l8", "f16", "f32"])
+@pytest.mark.parametrize("target", ["s8", "f16", "f32"])
+def test_srlab2_after_an_over_keeps_the_interpreters_bytes(ctx, source, target):
+    """'over' of two layers, to SrLab2 and back, alone and as a batch of two: the
+    chains that ran on the interpreter before they were compiled give its bytes."""
+    tex = {"s8": (W.RGBA8, z.Color.SRGB), "l8": (W.RGBA8, z.Color(transfer=z.Transfer.Linear)),
+           "f16": (W.RGBA16F, z.Color(transfer=z.Transfer.Linear)),
+           "f32": (z.Descriptor.rgba32f_linear(1, 1).texel, z.Color(transfer=z.Transfer.Linear))}
+    rng = np.random.default_rng(31)
+    for sizes in ([(257, 130)], [(257, 130), (61, 67)]):
+        cmd, inputs, host, outputs = z.CommandBuffer(), {}, {}, {}
+        for w, h in sizes:
+            d = z.Descriptor(w, h, *tex[source])
+            linear = []
+            for _ in range(2):
+                a = cmd.input(d)
+                inputs[a] = d
+                v = rng.random((h, w * 4))
+                host[a] = {"f16": v.astype(np.float16), "f32": v.astype(np.float32)}.get(
+                    source, (v * 256).astype(np.uint8)).view(np.uint8)
+                linear.append(cmd.color_convert(a, z.Color(transfer=z.Transfer.Linear), W.RGBA16F))
+            v = cmd.blend(linear[0], z.Rectangle(0, 0, w, h), linear[1])
+            lab = cmd.color_convert(v, z.Color.SRLAB2_D65, W.LABA16F)
+            o, od = cmd.output(cmd.color_convert(lab, tex[target][1], tex[target][0]))
+            outputs[o] = od
+        out, exe = run(ctx, cmd, inputs, host, outputs)
+        text = exe.describe()
+        assert "[kernel jit#" in text and "unavailable" not in text, text
+        ref, _ = run(ctx, cmd, inputs, host, outputs, flags=z.PLAN_INTERPRETER)
+        for o in outputs:
+            assert np.array_equal(out[o], ref[o])

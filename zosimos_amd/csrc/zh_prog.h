@@ -58,18 +58,21 @@ struct Prog {
     }
     return true;
   }
-  // SrLab2 programs round to FP32 before they round to half floats, as the
-  // interpreter does, so that an image gives the same bits with and without row
-  // padding (left visible, the last matrix's sums round to half floats at once).
-  static constexpr bool srlab() {
+  static constexpr bool holds(uint32_t op) {
     for (int k = 0; k < n; ++k)
-      if (el_op(el[k]) == OP_SRLAB || el_op(el[k]) == OP_SRLAB_INV) return true;
+      if (el_op(el[k]) == op) return true;
     return false;
   }
+  // SrLab2 programs give the interpreter's bits, which they ran on before they
+  // had kernels: an image comes out the same with and without row padding.
+  // Matrices sum in a written order, half-float stores round to FP32 first, a
+  // decoded 8-bit alpha is rounded before 1 - alpha is taken, and an 'over' is
+  // done in its steps.
+  static constexpr bool srlab() { return holds(OP_SRLAB) || holds(OP_SRLAB_INV); }
   // Elements i .. i + 4 composite a loaded layer over the value with straight
   // alpha in and out: premul, load (push), premul, over, unpremul.
   static constexpr bool straight_over(int i) {
-    return i + 4 < n && el_op(el[i]) == OP_PREMUL && el_op(el[i + 1]) == OP_LOAD && el_push(el[i + 1]) &&
+    return !srlab() && i + 4 < n && el_op(el[i]) == OP_PREMUL && el_op(el[i + 1]) == OP_LOAD && el_push(el[i + 1]) &&
            el_op(el[i + 2]) == OP_PREMUL && el_op(el[i + 3]) == OP_OVER && el_op(el[i + 4]) == OP_UNPREMUL;
   }
 };
@@ -230,14 +233,22 @@ __device__ __forceinline__ void exec(const Uni<P>& u, uint64_t x0, int n, const 
         for (int i = 0; i < kPix; ++i) { Z[i] = Y[i]; Y[i] = X[i]; }
       }
       decode<el_fmt(e)>(raw + P::woff(I), X, L);
+      if constexpr (P::srlab() && P::holds(OP_OVER)) {
+#pragma unroll
+        for (int i = 0; i < kPix; ++i) round_f32(X[i]);
+      }
     } else if constexpr (op == OP_MAT3) {
       const float* m = u.m + P::poff(I);
 #pragma unroll
       for (int i = 0; i < kPix; ++i) {
-        const float r = m[0] * X[i].x + m[1] * X[i].y + m[2] * X[i].z;
-        const float g = m[3] * X[i].x + m[4] * X[i].y + m[5] * X[i].z;
-        const float b = m[6] * X[i].x + m[7] * X[i].y + m[8] * X[i].z;
-        X[i] = make_float4(r, g, b, X[i].w);
+        if constexpr (P::srlab()) {
+          X[i] = make_float4(row3(m, X[i]), row3(m + 3, X[i]), row3(m + 6, X[i]), X[i].w);
+        } else {
+          const float r = m[0] * X[i].x + m[1] * X[i].y + m[2] * X[i].z;
+          const float g = m[3] * X[i].x + m[4] * X[i].y + m[5] * X[i].z;
+          const float b = m[6] * X[i].x + m[7] * X[i].y + m[8] * X[i].z;
+          X[i] = make_float4(r, g, b, X[i].w);
+        }
       }
     } else if constexpr (op == OP_CBRT && el_fmt(e) == 1) {  // input proved non-negative
       constexpr float t = 1.0f / 3.0f;
@@ -283,7 +294,7 @@ __device__ __forceinline__ void exec(const Uni<P>& u, uint64_t x0, int n, const 
       constexpr uint32_t F = el_fmt(e);
       if constexpr (F == FMT_F16 && P::srlab()) {
 #pragma unroll
-        for (int i = 0; i < kPix; ++i) asm volatile("" : "+v"(X[i].x), "+v"(X[i].y), "+v"(X[i].z));
+        for (int i = 0; i < kPix; ++i) round_f32(X[i]);
       }
       if constexpr (P::alpha_byte_passes()) {
         // Alpha bytes straight from the loaded texels (raw[0]: the 4 words).
