@@ -253,8 +253,8 @@ def test_c4_chain_small(ctx):
 
 def test_pointwise_batch_ragged(ctx):
     """Independent images of one pointwise signature run as one launch of the
-    batched kernel, in chunks of 16,384 pixels: sizes below, at and above a
-    chunk, with partial groups of 4 pixels.  The same executable then runs
+    batched kernel, in chunks of 1,024 pixels: sizes below and above a chunk and
+    of many, with partial groups of 4 pixels.  The same executable then runs
     with one image at an address that is not 16-byte aligned (each stage
     launches on its own), and aligned again (bit-identical to the first)."""
     sizes = [(1, 1), (3, 1), (7, 5), (128, 128), (129, 127), (300, 61), (16384, 1), (16385, 2)]

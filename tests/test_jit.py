@@ -23,17 +23,28 @@ def test_unregistered_chain_is_compiled_at_run_time():
     assert a == b
 
 
+def srlab_chain(out):
+    """SrLab2's encode of an RGBA8 image into half-float Lab, or of one with
+    linear texels (no registered signature)."""
+    d = z.Descriptor.rgba8_srgb(32, 32) if out == "registered" else z.Descriptor.rgba32f_linear(32, 32)
+    cmd = z.CommandBuffer()
+    cmd.output(cmd.color_convert(cmd.input(d), z.Color(model=z.ColorModel.SrLab2),
+                                 z.Texel(z.SampleBits.Float16x4, z.SampleParts.LabA)))
+    return cmd
+
+
 def test_registered_and_unsupported_chains():
     assert "[kernel c2_over" in describe(W.c2(64, 32).commands)
-    # SrLab2's encode is registered too
+    # SrLab2's encode is registered for RGBA8, and compiled for other texels
+    assert "[kernel srlab_enc_s8h]" in describe(srlab_chain("registered"))
+    assert "[kernel jit#" in describe(srlab_chain("linear"))
+    # no specialised body takes a channel apart
     d = z.Descriptor.rgba8_srgb(32, 32)
     cmd = z.CommandBuffer()
-    i = cmd.input(d)
-    s = cmd.color_convert(i, z.Color(model=z.ColorModel.SrLab2),
-                          z.Texel(z.SampleBits.Float16x4, z.SampleParts.LabA))
-    cmd.output(s)
+    a, b = cmd.input(d), cmd.input(d)
+    cmd.output(cmd.inject(a, z.ColorChannel.G, cmd.extract(b, z.ColorChannel.R)))
     text = describe(cmd)
-    assert "jit#" not in text
+    assert " channel " in text and "[kernel interp-inline]" in text and "jit#" not in text, text
 
 
 def test_tag_names_the_kernel_that_runs():

@@ -89,3 +89,50 @@ def test_static_launch_refuses_tables_beyond_the_scratch(ctx):
     got, _ = _static_run(ctx, wl, host)
     for o in ref:
         assert np.array_equal(got[o], ref[o])
+
+
+def test_static_launch_drops_tile_masks_for_space(ctx):
+    """Tables that fit the scratch only without the per-tile layer masks (2 bytes
+    a tile) are not refused: the largest buffer register that still launches
+    leaves less room than the masks take, and the output is the ordinary
+    program's."""
+    w, h = 1500, 1100  # 24 x 69 tiles: 3312 bytes of masks
+    d8 = z.Descriptor.rgba8_srgb(w, h)
+    rng = np.random.default_rng(35)
+    host = rng.integers(0, 256, (h, w * 4), dtype=np.uint8)
+    texels = rng.integers(0, 256, 32 << 20, dtype=np.uint8).tobytes()
+
+    def program(rows):  # a buffer register of `rows` rows of 64 texels, 256 bytes
+        cmd = z.CommandBuffer()
+        a = cmd.input(d8)
+        b = cmd.from_buffer(cmd.buffer_init(texels[:256 * rows]), z.Descriptor.rgba8_srgb(64, rows))
+        aff = W.about_centre(w, h, 0.7, 0.4)
+        o1, od1 = cmd.output(cmd.affine(cmd.solid_rgba(d8, (0, 0, 0, 0)), aff, a))
+        o2, od2 = cmd.output(b)
+        return cmd, a, {o1: od1, o2: od2}
+
+    img = ctx.image(d8)
+    img.upload(host)
+
+    def launch(rows):
+        cmd, a, outs = program(rows)
+        imgs = {o: ctx.image(d) for o, d in outs.items()}
+        z.Linker.from_included().compile(cmd).launch_static(ctx, {a: img}, imgs)
+        ctx.sync()
+        return [i.download() for i in imgs.values()]
+
+    lo, hi = 1, len(texels) // 256  # launches / is refused
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        try:
+            launch(mid)
+            lo = mid
+        except z.ZosimosError as e:
+            assert e.code == z.Status.OUT_OF_MEMORY
+            hi = mid
+    got = launch(lo)
+    cmd, a, outs = program(lo)
+    ref, exe = run(ctx, cmd, {a: d8}, {a: host}, outs)
+    assert "[kernel w_s8_s8]" in exe.describe()
+    for g, o in zip(got, outs):
+        assert np.array_equal(g, ref[o])
