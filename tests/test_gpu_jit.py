@@ -170,11 +170,11 @@ def test_two_half_float_sources_hold_their_registers(ctx, degrees):
 @pytest.mark.parametrize("degrees", [0.0, 12.0])
 @pytest.mark.parametrize("texel,w,h,few", [
     ("f16", 63, 15, True), ("f16", 400, 300, True), ("f16", 1024, 256, True), ("f16", 1025, 256, False),
-    ("f32", 63, 15, True), ("f32", 1025, 256, True), ("f32", 1400, 1400, False), ("u8", 400, 300, False)])
+    ("f32", 63, 15, False), ("f32", 1025, 256, False), ("f32", 1400, 1400, False), ("u8", 400, 300, False)])
 def test_compiled_form_of_few_tiles(ctx, texel, w, h, few, degrees):
     """Four layers through a compiled form: up to one tile per compute unit
-    (256) of half floats, or a grid resident as a whole of floats, the kernel
-    without a choice of path runs, else the other; within 1 code of the FP64
+    (256) of half floats the kernel without a choice of path runs, else the
+    form's other (floats have only kernels without one); within 1 code of the FP64
     oracle (colour where alpha is above 0.02)."""
     from oracle import color as C
     rng = np.random.default_rng([w, h])

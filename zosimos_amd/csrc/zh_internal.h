@@ -84,6 +84,7 @@ struct WarpForm {
   uint32_t src = 0, fmt = 0, mat = 0;
   std::vector<uint16_t> post;
   bool sep = false;
+  bool tables() const;  // does it code 8-bit sRGB?
 };
 // The form behind a StageDesc::variant (registered or run-time); false for none.
 bool warp_form_of(int variant, WarpForm* f);
@@ -266,8 +267,9 @@ struct zh_program {
   // Run-time kernels per stage (StagePlan::jit): stage form, that for few tiles
   // (or null), batch form, and their resident workgroups per CU.
   std::vector<hipFunction_t> jit_stage_fn, jit_few_fn, jit_batch_fn;
-  // Warp stages: tiles up to which the kernel for few runs (zh_warp_few_tiles).
-  std::vector<uint32_t> few_tiles;
+  // Warp stages: has the form a kernel for few tiles, and a grid without runs
+  // (warp_has_few, warp_has_runs)?
+  std::vector<uint8_t> few, persistent;
   std::vector<uint32_t> jit_resident, jit_batch_resident;
   // The stepped execution (zh_program_start_pool) still launching this
   // program's kernels; other launches wait for it to finish.

@@ -311,6 +311,13 @@ zh_status jit_warp_kernels(int id, bool sep, bool staged, int device, hipFunctio
   return st;
 }
 
+bool WarpForm::tables() const {
+  auto srgb8 = [](uint32_t f) { return f == FMT_U8_SRGB_RGBA || f == FMT_U8_SRGB_BGRA; };
+  bool any = srgb8(fmt);
+  for (uint16_t e : post) any = any || ((e & 0xffu) == OP_STORE && srgb8((e >> 8) & 0xfu));
+  return any;
+}
+
 bool warp_form_of(int variant, WarpForm* f) {
   if (variant < 0) return false;
   if (variant >= kJitWarpBase) {

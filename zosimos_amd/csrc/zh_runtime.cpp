@@ -33,7 +33,7 @@ hipError_t zh_launch_move(int words, const zh::StageDesc* d_dev, uint32_t width,
 hipError_t zh_launch_spec(int index, const zh::StageDesc* d_dev, uint32_t width, uint32_t height,
                           uint32_t cus, hipStream_t stream);
 hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, hipStream_t stream);
-void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int staged, uint32_t* blocks,
+void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int persistent, uint32_t* blocks,
                   uint32_t* run);
 hipError_t zh_launch_warp(int index, int staged, int few, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
                           uint32_t per_cu, hipStream_t stream);
@@ -615,12 +615,18 @@ static zh_status alloc_device(zh_program* p) {
   // be had leaves its stage on the interpreter, and the description says why.
   p->jit_stage_fn.assign(p->plan.stages.size(), nullptr);
   p->jit_few_fn.assign(p->plan.stages.size(), nullptr);
-  p->few_tiles.assign(p->plan.stages.size(), 0);
+  p->few.assign(p->plan.stages.size(), 0);
+  p->persistent.assign(p->plan.stages.size(), 0);
   p->jit_batch_fn.assign(p->plan.stages.size(), nullptr);
   p->jit_resident.assign(p->plan.stages.size(), 1);
   p->jit_batch_resident.assign(p->plan.stages.size(), 1);
   for (size_t s = 0; s < p->plan.stages.size(); ++s) {
     StagePlan& sp = p->plan.stages[s];
+    WarpForm form;
+    if (sp.desc.kind == STAGE_RESAMPLE && warp_form_of(sp.desc.variant, &form)) {
+      p->few[s] = warp_has_few(form.src, form.fmt) && !sp.staged;
+      p->persistent[s] = sp.staged || !warp_has_runs(form.src, form.fmt, form.tables());
+    }
     if (sp.desc.kind == STAGE_RESAMPLE && sp.desc.variant >= kJitWarpBase) {
       // A run-time warp form; without it the stage runs on the resample
       // interpreter, whose kernels accept the same tiles.
@@ -646,15 +652,7 @@ static zh_status alloc_device(zh_program* p) {
       p->jit_stage_fn[s] = f;
       p->jit_few_fn[s] = ff;
       p->jit_batch_fn[s] = fb;
-      WarpForm form;
-      if (ff && warp_form_of(sp.desc.variant, &form))
-        p->few_tiles[s] = zh_warp_few_tiles(form.src, form.fmt, p->jit_resident[s], (uint32_t)ctx->cus);
       continue;
-    }
-    if (sp.desc.kind == STAGE_RESAMPLE && sp.desc.variant >= 0 && !sp.staged) {
-      WarpForm form;
-      if (warp_form_of(sp.desc.variant, &form))
-        p->few_tiles[s] = zh_warp_few_tiles(form.src, form.fmt, zh_warp_resident(sp.desc.variant, 0), (uint32_t)ctx->cus);
     }
     if (sp.jit < 0) continue;
     std::string why;
@@ -811,7 +809,7 @@ zh_status zh_program_launch_bytes(zh_program* p, uint64_t* bytes, uint32_t max_l
 // Does warp stage s run its form's kernel for few tiles?
 static bool runs_few(const zh_program* p, size_t s) {
   const StageDesc& d = p->plan.stages[s].desc;
-  return s < p->few_tiles.size() && d.tiles_x * d.tiles_y <= p->few_tiles[s];
+  return s < p->few.size() && p->few[s] && d.tiles_x * d.tiles_y <= (uint32_t)p->ctx->cus;
 }
 
 // ", N bytes of scratch a lane" when one of the kernels spills registers.
@@ -1208,8 +1206,8 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
       if (p->plan.stages[u.ids[0]].desc.variant >= kJitWarpBase) {
         const uint32_t first = u.ids[0];
         uint32_t blocks, run;
-        zh_warp_grid(u.total_tiles, p->jit_batch_resident[first], (uint32_t)p->ctx->cus, u.blocks_per_cu, u.staged,
-                     &blocks, &run);
+        zh_warp_grid(u.total_tiles, p->jit_batch_resident[first], (uint32_t)p->ctx->cus, u.blocks_per_cu,
+                     p->persistent[first], &blocks, &run);
         if (blocks == 0) return ZH_OK;
         const BatchDesc* bd = u.d_batch;
         void* args[] = {&bd, &run};
@@ -1271,7 +1269,7 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
         // A run-time warp form: the grid and kernel of zh_launch_warp.
         const uint32_t tiles = sp.desc.tiles_x * sp.desc.tiles_y, cus = (uint32_t)p->ctx->cus;
         uint32_t blocks, run;
-        zh_warp_grid(tiles, p->jit_resident[first], cus, u.blocks_per_cu, sp.staged, &blocks, &run);
+        zh_warp_grid(tiles, p->jit_resident[first], cus, u.blocks_per_cu, p->persistent[first], &blocks, &run);
         if (blocks == 0) break;
         const hipFunction_t fn = runs_few(p, first) ? p->jit_few_fn[first] : p->jit_stage_fn[first];
         const StageDesc* dp = d;

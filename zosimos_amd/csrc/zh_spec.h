@@ -89,12 +89,29 @@ constexpr uint16_t sg(uint32_t op, uint32_t fmt = 0, uint32_t push = 0) {
 // X(name, source form, F, mat3 in the source program, post elements...)
 enum WarpSrc : uint32_t { WSRC_ONE = 0, WSRC_OVER2 = 1 };
 
-// Has a form a second stage kernel, without the choice of path by the host's
-// masks, for stages of few tiles?  There every instruction's latency shows (one
-// wave a SIMD), and border tests are cheaper than the choice: one source of half
-// floats or of floats.  Of 8-bit texels and of two sources the choice is as fast
-// or faster (four RGBA8 layers 400x300: 9.2 us against 9.4).
-constexpr bool warp_has_few(uint32_t src, uint32_t fmt) { return src == WSRC_ONE && (fmt == FMT_F16 || fmt == FMT_F32); }
+// Do a form's kernels skip the border tests of the tiles whose taps the host
+// found inside (the choice of a path per tile and layer)?  Not those of float
+// texels: they hold 110 registers and more, the choice costs as much as it saves
+// with one source (4 layers 400x300: 8.7 us, without 7.8; 3840x2160 128 and 129)
+// and more with two (4 layers 3840x2160: 242-254 us, without 230-233).
+constexpr bool warp_has_choice(uint32_t fmt) { return fmt != FMT_F32; }
+
+// Has a form a second stage kernel, without that choice, for stages of few
+// tiles?  There every instruction's latency shows (one wave a SIMD), and border
+// tests are cheaper: one source of half floats (8 layers 611x332, 210 tiles: 15.0
+// us against 15.9; 3 layers 1200x700, 874 tiles: 13.5 with the choice against
+// 13.9).  Of 8-bit texels and of two sources the choice is as fast or faster (four
+// RGBA8 layers 400x300: 9.2 us against 9.4).
+constexpr bool warp_has_few(uint32_t src, uint32_t fmt) { return src == WSRC_ONE && fmt == FMT_F16; }
+
+// Are a form's tiles dealt in runs (zh_warp_grid)?  Float texels only with one
+// source and without the 8-bit tables: 2 waves a SIMD of two sources end together
+// (3840x2160: 79-87 us, in runs 82-89), and the tables are loaded anew for each
+// run (one layer to RGBA8 at 3840x2160: 34-37 us, in runs 38-42; to RGBA32F 38-48,
+// in runs 35-45).
+constexpr bool warp_has_runs(uint32_t src, uint32_t fmt, bool tables) {
+  return fmt != FMT_F32 || (src == WSRC_ONE && !tables);
+}
 
 #define ZH_WARP_LIST(X)                                                                        \
   X(w_over2_s8, WSRC_OVER2, ZH_S8, 0, ZH_UP, ZH_ST(ZH_S8))                                      \
@@ -117,15 +134,6 @@ const char* zh_spec_name(int index);
 // for axis-aligned maps.
 int zh_warp_lookup(uint32_t src, uint32_t fmt, uint32_t mat, const uint16_t* post, int n);
 const char* zh_warp_name(int index);
-// Tiles up to which a stage of a form runs its kernel for few tiles (0: never),
-// `resident` workgroups of the other fitting a compute unit.  Half floats: one
-// tile per compute unit (8 layers 611x332, 210 tiles: 15.0 us against 15.9; 3
-// layers 1200x700, 874 tiles: 13.5 with the choice against 13.9).  Floats: while
-// the grid is resident as a whole (4 layers 400x300: 7.8 us against 8.7; 8 layers
-// 1200x700, 840 tiles: 32.8 against 34.6).
-uint32_t zh_warp_few_tiles(uint32_t src, uint32_t fmt, uint32_t resident, uint32_t cus);
-// Workgroups of warp kernel `index` that fit a compute unit.
-uint32_t zh_warp_resident(int index, int staged);
 // Does warp kernel `index` have an LDS-staged form (separable, one source)?
 int zh_warp_has_staged(int index);
 // The form of warp kernel `index` (source form, format, mat3 flag and post

@@ -18,7 +18,7 @@ __global__ __launch_bounds__(kBlock, min_waves<V>()) void k_warp(const StageDesc
   warp_stage<V>(dd, run);
 }
 
-// Stages of few tiles (zh_warp_few_tiles): the kernel without a choice of path.
+// Stages of at most one tile per compute unit: the kernel without a choice of path.
 template <class V>
 __global__ __launch_bounds__(kBlock) void k_warp_few(const StageDesc* dd, uint32_t run) {
   warp_stage<V, false>(dd, run);
@@ -39,6 +39,11 @@ template <class V>
 __global__ __launch_bounds__(kBlock) void k_warp_staged_batch(const BatchDesc* bb, uint32_t) {
   warp_staged_batch<V>(bb);
 }
+
+// The registered forms have runs: zh_launch_warp deals them all so.
+#define ZH_WARP_RUNS(name, src, f, mat, ...) static_assert(f != FMT_F32, #name);
+ZH_WARP_LIST(ZH_WARP_RUNS)
+#undef ZH_WARP_RUNS
 
 template <class V>
 constexpr void (*few_fn())(const StageDesc*, uint32_t) {
@@ -127,16 +132,14 @@ int zh_warp_has_staged(int index) {
 }
 
 // Grid of a warp launch over `tiles` tiles, `resident` workgroups fitting a
-// compute unit: blocks of run tiles for the dispatcher to balance (per_cu 0), or
-// a persistent grid (run 0): the staged kernels' pipelined loop; per_cu
-// workgroups per compute unit, which keeps more of each one's taps in the L1;
-// grids that are resident as a whole, where nothing is left to balance (two
-// 640x480 layers rotated, 300 tiles, 6.65 us against 7.67 in runs); and forms of
-// at most 2 waves a SIMD, whose shares end together (two RGBA32F sources at
-// 3840x2160: 87.3 us, in runs 91.2).
-void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int staged, uint32_t* blocks,
+// compute unit: blocks of run tiles for the dispatcher to balance, or a persistent
+// grid (run 0): where asked for (the staged kernels' pipelined loop, forms without
+// runs); per_cu workgroups per compute unit, which keeps more of each one's taps
+// in the L1; and grids that are resident as a whole, where nothing is left to
+// balance (two 640x480 layers rotated, 300 tiles, 6.65 us against 7.67 in runs).
+void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int persistent, uint32_t* blocks,
                   uint32_t* run) {
-  if (per_cu || staged || resident <= 2 || tiles <= resident * cus) {
+  if (per_cu || persistent || tiles <= resident * cus) {
     *run = 0;
     *blocks = std::min(tiles, (per_cu ? std::min(per_cu, resident) : resident) * cus);
     return;
@@ -152,28 +155,17 @@ void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_
   *blocks = (tiles + *run - 1) / *run;
 }
 
-uint32_t zh_warp_few_tiles(uint32_t src, uint32_t fmt, uint32_t resident, uint32_t cus) {
-  if (!zh::warp_has_few(src, fmt)) return 0;
-  return fmt == zh::FMT_F32 ? resident * cus : cus;
-}
-
-uint32_t zh_warp_resident(int index, int staged) {
-  if (index < 0 || index >= zh::spec::kNumWarps) return 0;
-  const auto& e = zh::spec::kWarps[index];
-  static uint32_t resident[2][zh::spec::kNumWarps] = {};
-  uint32_t& res = resident[staged ? 1 : 0][index];
-  if (!res) res = zh::resident_blocks((const void*)(staged ? e.staged : e.fn), 1);
-  return res;
-}
-
 hipError_t zh_launch_warp(int index, int staged, int few, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
                           uint32_t per_cu, hipStream_t stream) {
   if (index < 0 || index >= zh::spec::kNumWarps) return hipErrorInvalidValue;
   const auto& e = zh::spec::kWarps[index];
   const auto fn = staged ? e.staged : few ? e.few : e.fn;
   if (!fn) return hipErrorInvalidValue;
+  static uint32_t resident[2][zh::spec::kNumWarps] = {};
+  uint32_t& res = resident[staged ? 1 : 0][index];
+  if (!res) res = zh::resident_blocks((const void*)(staged ? e.staged : e.fn), 1);
   uint32_t blocks, run;
-  zh_warp_grid(tiles, zh_warp_resident(index, staged), cus, per_cu, staged, &blocks, &run);
+  zh_warp_grid(tiles, res, cus, per_cu, staged, &blocks, &run);
   if (blocks == 0) return hipSuccess;
   hipLaunchKernelGGL(fn, dim3(blocks), dim3(zh::kBlock), 0, stream, d_dev, run);
   return hipGetLastError();

@@ -434,7 +434,7 @@ __device__ __forceinline__ void layer_taps(const LayerArgs& a, const LaneMap& mp
 // lane (lx, ly) owns pixels x = tx * tile_w + lx + k * lanes_x (k < kPix) of
 // row ty * tile_h + ly, so every load and store instruction covers runs of
 // lanes_x adjacent pixels.
-template <class V, bool INSIDE = true>
+template <class V, bool INSIDE = warp_has_choice(V::F)>
 __device__ __forceinline__ void warp_tile(CDesc d, uint32_t tx, uint32_t ty, const Luts* L) {
   typedef typename V::Post Post;
   typedef typename RawT<V::F>::type R;
@@ -871,7 +871,7 @@ __device__ __forceinline__ Deal deal_tiles(uint32_t total, uint32_t run) {
 template <class V>
 constexpr int min_waves() { return V::F == FMT_F16 && V::SRC == WSRC_ONE ? 5 : 1; }
 
-template <class V, bool INSIDE = true>
+template <class V, bool INSIDE = warp_has_choice(V::F)>
 __device__ __forceinline__ void warp_stage(const StageDesc* dd, uint32_t run) {
   const CDesc d = as_const(dd);
   __shared__ Luts luts;
