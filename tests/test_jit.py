@@ -4,6 +4,7 @@ ZH_PLAN_NO_JIT asks for the interpreter; registered chains keep their
 kernels, and chains with operations the specialised bodies lack stay on the
 interpreter."""
 import ctypes
+import itertools
 
 import zosimos_amd as z
 from zosimos_amd import workloads as W
@@ -79,22 +80,24 @@ def test_unregistered_warp_form_is_compiled_at_run_time():
     assert "_sep_lds]" in describe(cmd2, z.PLAN_STAGED).split("jitw#")[1]
 
 
-def _warp_grid(tiles, resident, cus=256, per_cu=0, persistent=0):
+def _warp_grid(tiles, resident, cus=256, per_cu=0, persistent=0, layers=0):
     blocks, run = ctypes.c_uint32(), ctypes.c_uint32()
     z._abi.lib().zh_warp_grid(*map(ctypes.c_uint32, (tiles, resident, cus, per_cu)), ctypes.c_int(persistent),
-                              ctypes.byref(blocks), ctypes.byref(run))
+                              ctypes.c_uint32(layers), ctypes.byref(blocks), ctypes.byref(run))
     return blocks.value, run.value
 
 
 def test_warp_grids_cover_their_tiles():
     """Runs of tiles for grids past the resident one: every tile in one run, no
     empty workgroup."""
-    for resident in (1, 2, 3, 5, 7):
+    for resident, layers in itertools.product((1, 2, 3, 5, 7), (0, 1, 2, 8)):
         for tiles in (1, 255, 256 * resident, 256 * resident + 1, 8160, 100_003, 10_000_019):
-            blocks, run = _warp_grid(tiles, resident)
+            blocks, run = _warp_grid(tiles, resident, layers=layers)
             if tiles <= 256 * resident:
                 assert run == 0 and blocks == tiles
             else:
                 assert 1 <= run <= 8 and (blocks - 1) * run < tiles <= blocks * run
+    # tables and one layer: two tiles a run
+    assert [_warp_grid(8160, 5, layers=n)[1] for n in (0, 1, 2)] == [1, 2, 1]
     assert _warp_grid(100_000, 6, per_cu=2) == (512, 0)
     assert _warp_grid(100_000, 6, persistent=1) == (1536, 0)

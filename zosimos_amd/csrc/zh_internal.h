@@ -267,9 +267,9 @@ struct zh_program {
   // Run-time kernels per stage (StagePlan::jit): stage form, that for few tiles
   // (or null), batch form, and their resident workgroups per CU.
   std::vector<hipFunction_t> jit_stage_fn, jit_few_fn, jit_batch_fn;
-  // Warp stages: has the form a kernel for few tiles, and a grid without runs
-  // (warp_has_few, warp_has_runs)?
-  std::vector<uint8_t> few, persistent;
+  // Warp stages: has the form a kernel for few tiles, a grid without runs
+  // (warp_has_few, warp_has_runs), the 8-bit tables?
+  std::vector<uint8_t> few, persistent, tables;
   std::vector<uint32_t> jit_resident, jit_batch_resident;
   // The stepped execution (zh_program_start_pool) still launching this
   // program's kernels; other launches wait for it to finish.

@@ -33,10 +33,10 @@ hipError_t zh_launch_move(int words, const zh::StageDesc* d_dev, uint32_t width,
 hipError_t zh_launch_spec(int index, const zh::StageDesc* d_dev, uint32_t width, uint32_t height,
                           uint32_t cus, hipStream_t stream);
 hipError_t zh_launch_spec_batch(int index, const zh::BatchDesc* b_dev, uint32_t total_chunks, hipStream_t stream);
-void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int persistent, uint32_t* blocks,
-                  uint32_t* run);
-hipError_t zh_launch_warp(int index, int staged, int few, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
-                          uint32_t per_cu, hipStream_t stream);
+void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int persistent, uint32_t layers,
+                  uint32_t* blocks, uint32_t* run);
+hipError_t zh_launch_warp(int index, int staged, int few, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t layers,
+                          uint32_t cus, uint32_t per_cu, hipStream_t stream);
 hipError_t zh_launch_warp_batch(int index, int staged, const zh::BatchDesc* b_dev, uint32_t total_tiles,
                                 uint32_t cus, uint32_t per_cu, hipStream_t stream);
 hipError_t zh_launch_resample(const zh::StageDesc* d_dev, int mode, uint32_t tiles_x, uint32_t tiles_y,
@@ -617,6 +617,7 @@ static zh_status alloc_device(zh_program* p) {
   p->jit_few_fn.assign(p->plan.stages.size(), nullptr);
   p->few.assign(p->plan.stages.size(), 0);
   p->persistent.assign(p->plan.stages.size(), 0);
+  p->tables.assign(p->plan.stages.size(), 0);
   p->jit_batch_fn.assign(p->plan.stages.size(), nullptr);
   p->jit_resident.assign(p->plan.stages.size(), 1);
   p->jit_batch_resident.assign(p->plan.stages.size(), 1);
@@ -625,6 +626,7 @@ static zh_status alloc_device(zh_program* p) {
     WarpForm form;
     if (sp.desc.kind == STAGE_RESAMPLE && warp_form_of(sp.desc.variant, &form)) {
       p->few[s] = warp_has_few(form.src, form.fmt) && !sp.staged;
+      p->tables[s] = form.tables();
       p->persistent[s] = sp.staged || !warp_has_runs(form.src, form.fmt, form.tables());
     }
     if (sp.desc.kind == STAGE_RESAMPLE && sp.desc.variant >= kJitWarpBase) {
@@ -810,6 +812,11 @@ zh_status zh_program_launch_bytes(zh_program* p, uint64_t* bytes, uint32_t max_l
 static bool runs_few(const zh_program* p, size_t s) {
   const StageDesc& d = p->plan.stages[s].desc;
   return s < p->few.size() && p->few[s] && d.tiles_x * d.tiles_y <= (uint32_t)p->ctx->cus;
+}
+
+// Layers of warp stage s when its kernel loads the 8-bit tables (zh_warp_grid).
+static uint32_t table_layers(const zh_program* p, size_t s) {
+  return s < p->tables.size() && p->tables[s] ? p->plan.stages[s].desc.n_layers : 0u;
 }
 
 // ", N bytes of scratch a lane" when one of the kernels spills registers.
@@ -1207,7 +1214,7 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
         const uint32_t first = u.ids[0];
         uint32_t blocks, run;
         zh_warp_grid(u.total_tiles, p->jit_batch_resident[first], (uint32_t)p->ctx->cus, u.blocks_per_cu,
-                     p->persistent[first], &blocks, &run);
+                     p->persistent[first], 0, &blocks, &run);
         if (blocks == 0) return ZH_OK;
         const BatchDesc* bd = u.d_batch;
         void* args[] = {&bd, &run};
@@ -1269,7 +1276,8 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
         // A run-time warp form: the grid and kernel of zh_launch_warp.
         const uint32_t tiles = sp.desc.tiles_x * sp.desc.tiles_y, cus = (uint32_t)p->ctx->cus;
         uint32_t blocks, run;
-        zh_warp_grid(tiles, p->jit_resident[first], cus, u.blocks_per_cu, p->persistent[first], &blocks, &run);
+        zh_warp_grid(tiles, p->jit_resident[first], cus, u.blocks_per_cu, p->persistent[first], table_layers(p, first),
+                     &blocks, &run);
         if (blocks == 0) break;
         const hipFunction_t fn = runs_few(p, first) ? p->jit_few_fn[first] : p->jit_stage_fn[first];
         const StageDesc* dp = d;
@@ -1277,7 +1285,7 @@ static zh_status launch_unit(zh_program* p, const Unit& u) {
         ZH_HIP(hipModuleLaunchKernel(fn, blocks, 1, 1, kBlock, 1, 1, 0, s, args, nullptr));
       } else if (first < p->variant.size() && p->variant[first] == 3) {
         ZH_HIP(zh_launch_warp(sp.desc.variant, sp.staged, runs_few(p, first), d, sp.desc.tiles_x * sp.desc.tiles_y,
-                              (uint32_t)p->ctx->cus, u.blocks_per_cu, s));
+                              table_layers(p, first), (uint32_t)p->ctx->cus, u.blocks_per_cu, s));
       } else if (first < p->variant.size() && p->variant[first] == 9) {
         ZH_HIP(zh_launch_move(sp.move, d, sp.desc.width, sp.desc.height, s));
       } else {

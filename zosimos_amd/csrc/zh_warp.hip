@@ -137,8 +137,9 @@ int zh_warp_has_staged(int index) {
 // runs); per_cu workgroups per compute unit, which keeps more of each one's taps
 // in the L1; and grids that are resident as a whole, where nothing is left to
 // balance (two 640x480 layers rotated, 300 tiles, 6.65 us against 7.67 in runs).
-void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int persistent, uint32_t* blocks,
-                  uint32_t* run) {
+// layers: of a stage whose kernel loads the 8-bit tables (0: none or a batch).
+void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_cu, int persistent, uint32_t layers,
+                  uint32_t* blocks, uint32_t* run) {
   if (per_cu || persistent || tiles <= resident * cus) {
     *run = 0;
     *blocks = std::min(tiles, (per_cu ? std::min(per_cu, resident) : resident) * cus);
@@ -152,11 +153,16 @@ void zh_warp_grid(uint32_t tiles, uint32_t resident, uint32_t cus, uint32_t per_
   // (6 tiles per resident workgroup), run 1 / 2 / 4: 132 / 134 / 149 us,
   // persistent 150.
   *run = std::max(1u, std::min(8u, tiles / (12u * resident * cus)));
+  // A run loads the tables anew, which one layer's taps do not hide: two tiles a
+  // run from 2.5 per resident workgroup on (one RGBA16F layer to RGBA8 at 3840x2160,
+  // 6.4: 35.4-36.6 us, in twos 32.3-33.8; 2560x1440, 2.8: 19.1 and 18.3-18.5).  Two
+  // layers gain or lose by the map (3840x2160 RGBA8 49.6 and 50.9).
+  if (layers == 1 && (uint64_t)tiles * 2 >= (uint64_t)resident * cus * 5) *run = std::max(*run, 2u);
   *blocks = (tiles + *run - 1) / *run;
 }
 
-hipError_t zh_launch_warp(int index, int staged, int few, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t cus,
-                          uint32_t per_cu, hipStream_t stream) {
+hipError_t zh_launch_warp(int index, int staged, int few, const zh::StageDesc* d_dev, uint32_t tiles, uint32_t layers,
+                          uint32_t cus, uint32_t per_cu, hipStream_t stream) {
   if (index < 0 || index >= zh::spec::kNumWarps) return hipErrorInvalidValue;
   const auto& e = zh::spec::kWarps[index];
   const auto fn = staged ? e.staged : few ? e.few : e.fn;
@@ -165,7 +171,7 @@ hipError_t zh_launch_warp(int index, int staged, int few, const zh::StageDesc* d
   uint32_t& res = resident[staged ? 1 : 0][index];
   if (!res) res = zh::resident_blocks((const void*)(staged ? e.staged : e.fn), 1);
   uint32_t blocks, run;
-  zh_warp_grid(tiles, res, cus, per_cu, staged, &blocks, &run);
+  zh_warp_grid(tiles, res, cus, per_cu, staged, layers, &blocks, &run);
   if (blocks == 0) return hipSuccess;
   hipLaunchKernelGGL(fn, dim3(blocks), dim3(zh::kBlock), 0, stream, d_dev, run);
   return hipGetLastError();
@@ -181,7 +187,7 @@ hipError_t zh_launch_warp_batch(int index, int staged, const zh::BatchDesc* b_de
   uint32_t& res = resident[staged ? 1 : 0][index];
   if (!res) res = zh::resident_blocks((const void*)fn, 1);
   uint32_t blocks, run;
-  zh_warp_grid(total_tiles, res, cus, per_cu, staged, &blocks, &run);
+  zh_warp_grid(total_tiles, res, cus, per_cu, staged, 0, &blocks, &run);
   if (blocks == 0) return hipSuccess;
   hipLaunchKernelGGL(fn, dim3(blocks), dim3(zh::kBlock), 0, stream, b_dev, run);
   return hipGetLastError();
