@@ -78,18 +78,22 @@ def test_box3_transfers(ctx, bits, transfer):
 
 
 # Octaves past the cached ones, cells smaller than a pixel (nothing fits the
-# cache, or only the low octaves), several tiles with ragged edges, an
-# octave count of 0.
-@pytest.mark.parametrize("w,h,octaves,scale", [(64, 16, 3, (7.0, 5.0)), (131, 37, 12, (3.0, 8.0)),
-                                               (65, 17, 2, (4000.0, 3.0)), (200, 50, 5, (150.0, 90.0)),
-                                               (70, 20, 4, (1e6, 1e6)), (3, 2, 0, (5.0, 5.0))])
-def test_noise_cache(ctx, w, h, octaves, scale):
+# cache, or only the low octaves), several tiles with ragged edges, an octave
+# count of 0; and images of so few tiles (under 1024) and so many corners that
+# they stay on the interpreter.
+@pytest.mark.parametrize("w,h,octaves,scale,kernel", [
+    (2560, 410, 3, (280.0, 130.0), True), (2553, 415, 12, (70.0, 90.0), True), (2561, 401, 2, (150000.0, 80.0), True),
+    (1600, 660, 5, (1200.0, 900.0), True), (2000, 520, 4, (1e6, 1e6), True), (3, 2, 0, (5.0, 5.0), True),
+    (64, 16, 3, (7.0, 5.0), False), (131, 37, 12, (3.0, 8.0), False), (65, 17, 2, (4000.0, 3.0), False),
+    (200, 50, 5, (150.0, 90.0), False), (70, 20, 4, (1e6, 1e6), False), (64, 16, 1, (7.0, 5.0), True),
+    (331, 137, 3, (7.0, 5.0), True)])
+def test_noise_cache(ctx, w, h, octaves, scale, kernel):
     """The noise's values are a fixed function of f32 arithmetic: bit-exact."""
     n = z.FractalNoise(octaves, 0.25, 0.75, scale)
     cmd = z.CommandBuffer()
     o, od = cmd.output(cmd.distribution_fractal_noise(z.Descriptor.rgba32f_linear(w, h), n))
     out, exe = run_both(ctx, cmd, {}, {}, {o: od})
-    assert "field kernel" in exe.describe()
+    assert ("field kernel" in exe.describe()) == kernel
     want = PL.fractal_noise(w, h, octaves, n.initial_amplitude, n.amplitude_damping, scale).astype(np.float32)
     assert np.array_equal(out[o].view(np.float32).reshape(h, w, 4), want)
 

@@ -159,7 +159,7 @@ __device__ __forceinline__ float4 grid_value(CParams q, float u, float v) {
 // corner per lane, in batches of the octaves that fit the cache together, with
 // the difference to the corner below that the blend takes; the hash is 10
 // quarter-rate multiplies a corner, four corners a pixel and octave without the
-// cache: 92 us for four octaves at 2048x2048, 45 with it, bound by the blend's
+// cache: 92 us for four octaves at 2048x2048, 50 with it, bound by the blend's
 // vector instructions.  Octaves whose box does not fit (cells smaller than a
 // pixel) hash directly, as does a lane with a pixel whose rounded coordinate
 // falls outside the box.

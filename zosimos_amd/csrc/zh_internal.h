@@ -112,6 +112,7 @@ struct StagePlan {
   int jit = -1;                   // pointwise: run-time kernel of the signature (zh_jit.cpp), -1 = none
   int any = -1;                   // pointwise: shape of the any-format kernels (zh_any.hip), -1 = none
   int field = -1;                 // pointwise: shape of the kernels of zh_field.hip, -1 = none
+  bool field_pays = true;         // and that is faster than the interpreter (noise_pays)
   int move = 0;                   // resample: 32-bit words of a texel k_move moves (zh_move.hip), 0 = not its form
   bool staged = false;            // warp: the LDS-staged kernel (staged_tile), the box fitting its tile
   uint32_t lds_bytes = 0;

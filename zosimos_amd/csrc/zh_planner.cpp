@@ -1191,6 +1191,29 @@ static int field_shape(StageDesc& d) {
   return (int)shape;
 }
 
+// Does the noise stage run k_noise (zh_field.hip) rather than the interpreter?  Its
+// workgroups hash a tile's corners in batches, one after the other, which only
+// many workgroups hide: from 4 tiles of 64 x 16 a compute unit on, or where every
+// octave's corners (about as many as the tile has cells, and three more a side)
+// are few enough for one short batch.  Five octaves of 37 x 21 cells: 250x200 17.5
+// us, the interpreter 12.0; four 1200x900 (1083 tiles) 17 and 30; two 500x400 (110
+// corners) 7.0 and 7.9; one of 150 x 120 cells 250x200 (521 corners) 9.8 and 6.9,
+// 500x400 (173) 5.7 and 6.6.
+static bool noise_pays(const StageDesc& d) {
+  const uint64_t tiles = (uint64_t)((d.width + 63) / 64) * ((d.height + 15) / 16);
+  if (tiles >= 1024) return true;
+  const float* q = d.params + d.code[0].arg;
+  const double dx = std::min(64.0 / d.width, 1.0), dy = std::min(16.0 / d.height, 1.0);
+  double corners = 0.0;
+  for (int k = 0; (float)k < q[4]; ++k) {
+    // Octave k is the first turned by k / 2 and scaled by 2^k.
+    const double c = std::fabs(std::ldexp(std::cos(0.5 * k), k)), s = std::fabs(std::ldexp(std::sin(0.5 * k), k));
+    corners += ((c * dx + s * dy) * std::fabs(q[0]) + 3.0) * ((s * dx + c * dy) * std::fabs(q[1]) + 3.0);
+    if (!(corners <= 400.0)) return false;
+  }
+  return true;
+}
+
 // Shape of the any-format kernels the pointwise program has (AnyShape), its
 // decode tables set; -1 for any other program.
 static int any_shape(StageDesc& d, bool flat) {
@@ -1233,7 +1256,7 @@ int pointwise_variant(const StagePlan& sp, bool jit, bool aligned, bool natural)
   if (aligned && sp.spec >= 0) return 2;
   if (aligned && jit) return 6;
   if (natural && sp.any >= 0) return 7;
-  if (natural && sp.field >= 0) return 8;
+  if (natural && sp.field >= 0 && sp.field_pays) return 8;
   return aligned && sp.fast ? 1 : 0;
 }
 
@@ -1649,6 +1672,7 @@ zh_status plan_program(const std::vector<zh_descriptor>& textures, const std::ve
       if (!interpreter) {
         sp.any = any_shape(sp.desc, flat);
         if (!flat && sp.any < 0) sp.field = field_shape(sp.desc);
+        if (sp.field >= 0 && field_kind((uint32_t)sp.field) == FIELD_NOISE) sp.field_pays = noise_pays(sp.desc);
       }
       for (size_t k = 0; k < sp.slot_ref.size(); ++k)
         if (sp.slot_ref[k] > -1000000 || sp.slot_ref[k] < -2000000000ll) {
